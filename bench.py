@@ -142,13 +142,16 @@ def cpu_baseline(setup, state, n0, nsteps, budget_s):
     return out
 
 
-def profiled_traffic(kernel_class: str, workload: str, sor_rows: int = 4):
+def profiled_traffic(kernel_class: str, workload: str, sor_rows: int = 4, resident: bool = False):
     """HBM bytes per launch of the dominant kernel, as measured by the
     rocprofv3 FETCH_SIZE and WRITE_SIZE counters (scaled by a copy of known
     size) and recorded in profiles/<kernel>_<workload>.md; None when no such
     measurement is recorded for this kernel and workload.  sor_rows: the SOR
-    kernel in use (4 two iterations per launch, 2 or 1 one)."""
-    if kernel_class == "sor":
+    kernel in use (4 two iterations per launch, 2 or 1 one); resident: all
+    iterations in one launch."""
+    if kernel_class == "sor" and resident:
+        name = "sor_res"
+    elif kernel_class == "sor":
         if os.environ.get("LES_SOR_FUSED", "1") == "0":
             name = "sor_sweep"
         else:
@@ -554,12 +557,17 @@ def main(argv=None):
     avg_s = dom_ms / 1e3 / dom_n
     alg_bytes = CLASS_BYTES.get(dom_cls, 0) * w.cells
     fused = os.environ.get("LES_SOR_FUSED", "1") != "0"
+    # one launch per step and no class "sor1": all iterations in one launch
+    resident = kt.get("sor1", (0.0, 0))[1] == 0 and kt["sor"][1] == K and L > 1
     # SOR iterations per launch: 2 for the two-iteration kernel (the tuned or
     # default shape reports rows 4), 1 for one fused iteration, 1/2 for the
     # colour sweeps (LES_SOR_FUSED=0)
     sor_rows = (tuned or {}).get("rows", 4)  # untuned: the default shape (two iterations per launch)
     ipl = 0.5 if not fused else (2 if sor_rows == 4 else 1)
-    if dom_cls == "sor":
+    if dom_cls == "sor" and resident:
+        ipl = sum(iters_run) / dom_n
+        alg_bytes = SOR_BYTES_PER_ITER * w.cells * ipl
+    elif dom_cls == "sor":
         # Class "sor" holds the SOR launches after the one holding iteration
         # 1 (class "sor1"), or all colour sweeps (LES_SOR_FUSED=0).
         # Launches after a step's stop test exit at once: the iterations
@@ -571,7 +579,7 @@ def main(argv=None):
         avg_s = dom_ms / 1e3 / max(1, round(iters / ipl))
     in_step_us = avg_s * 1e6
     timing_method = "one HIP event pair per launch in K eager steps"
-    if dom_cls == "sor" and fused and round(iters / ipl) == dom_n:
+    if dom_cls == "sor" and fused and not resident and round(iters / ipl) == dom_n:
         # every launch carried its iterations: the kernel's duration from
         # SOR_RUN back-to-back iterations of the same kernel and launch shape
         # on the domain's stream between one event pair (les_domain_time_sor
@@ -609,7 +617,7 @@ def main(argv=None):
             "peak": HBM_PEAK_GBS,
             "unit": "GB/s",
             "frac": round(achieved / HBM_PEAK_GBS, 4),
-            "traffic": profiled_traffic(dom_cls, w.name, sor_rows),
+            "traffic": profiled_traffic(dom_cls, w.name, sor_rows, resident),
             "alg_bytes_per_launch": int(alg_bytes),
             "sor_iterations_per_launch": ipl if dom_cls == "sor" else None,
             "avg_launch_us": round(avg_s * 1e6, 3),
@@ -618,13 +626,16 @@ def main(argv=None):
         },
         "kernels": per_kernel,
     }
-    if tuned is not None:
+    if resident:
+        result["sor_launch"] = {"kernel": "k_sor_res (all iterations of a press in one launch)"}
+    elif tuned is not None:
         result["sor_launch"] = {"kernel": {4: "k_sor_pair (two iterations per launch)",
                                            2: "k_sor_iter2", 1: "k_sor_iter"}[tuned["rows"]],
                                 "rows_per_thread": min(tuned["rows"], 2), "tile_rows": tuned["tile_rows"],
                                 "tile_pairs": tuned["tile_width"], "k_levels_per_block": tuned["kchunk"],
                                 "tuned_us_per_iter": round(tuned["us_per_iter"], 2),
                                 "default_us_per_iter": round(tuned["us_per_iter_default"], 2)}
+    if tuned is not None:
         result["stencil_launch"] = {"k_levels_per_thread": {"velfg_feedbf": tuned["velfg_kchunk"],
                                                             "les_sm": tuned["sm_kchunk"],
                                                             "les_visc_adam": tuned["visc_kchunk"]},

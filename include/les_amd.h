@@ -251,8 +251,9 @@ int les_domain_stencil_chunks(les_domain* d, int* velfg_kchunk, int* sm_kchunk, 
  * up to whole launches): `iters` back-to-back iterations (numbered 2.., never stopping) on
  * the domain's SOR scratch arrays between one pair of HIP events on its
  * stream.  Leaves the fields and the last press statistics unchanged;
- * synchronises.  No reference counterpart: the measurement of the dominant
- * kernel. */
+ * synchronises.  It times the kernels that run one or two iterations per
+ * launch, also on a domain whose press solves in one launch.  No reference
+ * counterpart: the measurement of the dominant kernel. */
 int les_domain_time_sor(les_domain* d, int iters, double* us_per_iter);
 /* With on != 0, steps n > 1 replay one captured HIP graph of the whole
  * step (recaptured when the domain's constants change); results are the

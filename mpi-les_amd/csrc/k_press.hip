@@ -305,6 +305,7 @@ __global__ __launch_bounds__(256) void k_finalize_head(const double* __restrict_
   if (threadIdx.x == 0) {
     ctrl->rhsav = s / denom;
     ctrl->p_ghost_diff = fl != 0.0 ? 1 : 0;
+    res_begin(ctrl);
   }
 }
 
@@ -2515,7 +2516,8 @@ void launch_press(const DevDomain& d, float dt) {
   const int nred = gx * gy * gz;
   SplitBufs sb = d.sb;
   if (d.cn1_separable) sb.cn1[0] = sb.cn1[1] = nullptr;
-  if (d.press_mode == 0 && d.sor_fused && d.nmaxp >= 1 && sor_shape(d).rows == 4) {
+  const bool res = d.press_mode == 0 && d.nmaxp >= 1 && use_res(d);
+  if (res || (d.press_mode == 0 && d.sor_fused && d.nmaxp >= 1 && sor_shape(d).rows == 4)) {
     // two iterations per launch: the head in one pass (k_rhs_head), the mean
     // removal over the split rhs alone (k_rhs_sub); the launch of iterations
     // 1 and 2 reads the entry ghosts of p where they differ from their boundp
@@ -2529,6 +2531,11 @@ void launch_press(const DevDomain& d, float dt) {
     const long n4 = (long)s.cplane * g.km / 2;  // both colours, four floats at a time
     TIMED(d, KC_RHS, hipLaunchKernelGGL(k_rhs_sub, dim3(kRhsSubBlocks), dim3(256), 0, d.stream,
                                         (const float4*)sb.rhsr[0], (float4*)sb.rhs[0], n4, (const Ctrl*)d.ctrl));
+    if (res) {  // the whole solve in one launch
+      launch_sor_res(d, sb, d.nmaxp, d.pjuge, d.omega, false);
+      launch_press_mean(d, sb, gx, gy, gz, nred);
+      return;
+    }
     const PairLaunch last = launch_sor_pairs(d, sb, h, d.pjuge, 1, d.nmaxp, 0, d.F.p);
     TIMED(d, KC_PAV, hipLaunchKernelGGL(k_sor_pair_final, dim3(1), dim3(256), 0, d.stream, sb, d.ctrl, last,
                                         h.nparts, d.pjuge));

@@ -1,0 +1,893 @@
+// The red-black SOR of press (press.f95:89-122) as one launch per solve: the
+// iterates and the right-hand side stay in the registers of the whole GPU
+// from the first iteration to the last.
+//
+// A domain is cut into nb boxes of pairs x rows x levels, one per block and
+// at most one block per compute unit.  A thread owns one (pair, row) column
+// of its box -- red and black cell of each level, their rhs, in registers --
+// so the k neighbours are its own values; the in-plane neighbours come from
+// one LDS copy of the colour last updated, with a ring of halo cells around
+// it.  After each colour sweep the blocks exchange the cells on their box
+// faces through memory as 8-byte {value, tag} words (relaxed agent-scope
+// atomics: a word whose tag is the expected sweep carries the value, so no
+// flag, fence or second round trip is needed).  Every update is k_sor_pair's
+// expression on the same operands, so the iterates have the same bits.
+//
+// What bounds it: the exchange on small domains (one word crosses between two
+// compute units in 1 us, and a solve of 50 iterations waits for 100 of them
+// in a row), the vector ALU on large ones (19 instructions per cell, four
+// waves per SIMD; at 300x300x90 about 4 us of each 7.8 us sweep).  The
+// launches per two iterations it replaces where a domain fits (k_sor_pair)
+// cost 8 us each on the smallest domains and recompute a four-cell ring and
+// six extra levels per block on large ones (0.37 of their lane-steps are
+// useful at 300x300x90).  Microseconds of a 50-iteration solve, before and
+// now: 24x20x16 455 and 196, 96x96x64 498 and 242, 150x150x90 675 and 341,
+// 203x117x61 878 and 329 (odd jm: one iteration per launch before), 300x300x90
+// 1130 and 790.
+//
+// Waiting on other blocks is safe only while all of them run.  The blocks
+// first count themselves in (res_enter).  When all have arrived, none can be
+// left unscheduled and the waits always end.  When they have not within
+// kEnterTicks (another process's blocks hold the compute units), the launch
+// falls back to sweeps over memory handed out by a ticket counter
+// (res_ticket): a sweep waits only for tickets taken earlier, which running
+// blocks hold, so that needs no co-residency at all.
+#include <algorithm>
+#include <type_traits>
+
+#include "les_kernels.h"
+
+namespace les {
+
+namespace {
+
+typedef unsigned long long u64;
+// Two kernels: one block per compute unit with 256 registers a thread, and two
+// blocks per unit with 128.  With two, one box computes while the other waits
+// for its halo; with one, the box is larger (fewer faces) and the loads of four
+// levels are in flight at a time.  per: blocks per unit; plane: floats per
+// level of the LDS copy (a box and its halo ring, and a cell nothing reads),
+// at most; words: in-plane halo words per thread, at most; levels: of a box
+// (two to four registers each), at most; group: levels fetched together.
+constexpr int kResNT = 512;  // threads per block, at most
+struct ResClass {
+  int per, plane, words, levels, group;
+};
+constexpr ResClass kResClass[2] = {{1, 832, 8, 40, 4}, {2, 640, 4, 24, 2}};
+// Levels whose black rhs lies in LDS beside the copy instead of in registers.
+constexpr int res_lds_rhs(int cls, int bk) {
+  const int room = (163840 / kResClass[cls].per - 512 - 4 * bk * kResClass[cls].plane) / (4 * kResNT);
+  return cls == 0 ? 0 : room < bk ? room : bk;
+}
+constexpr long long kEnterTicks = 100000;  // 1 ms of the 100 MHz wall clock
+constexpr int kSpinMax = 1 << 22;  // polls of one word before the solve is given up (seconds)
+
+__device__ __forceinline__ int rcix(const SplitGrid& s, int t, int j, int k) {
+  return t + (j - 1) * s.cp + (k - 1) * s.cplane;
+}
+
+template <class T>
+__device__ __forceinline__ T ald(const T* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <class T>
+__device__ __forceinline__ void ast(T* p, T v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ u64 word(unsigned tag, float v) { return ((u64)tag << 32) | __float_as_uint(v); }
+__device__ __forceinline__ unsigned wtag(u64 w) { return (unsigned)(w >> 32); }
+__device__ __forceinline__ float wval(u64 w) { return __uint_as_float((unsigned)w); }
+// A table no kernel running beside this one writes: uniform reads of it are
+// scalar loads whatever the kernel stores in between.
+typedef const __attribute__((address_space(4))) float* ConstF;
+__device__ __forceinline__ ConstF constf(const float* p) { return (ConstF)(unsigned long long)p; }
+
+// The solve's arguments, read again where they are used (scalar loads from
+// the scalar cache): held over the solve they would take most of the scalar
+// registers, and the rest would spill into vector ones.
+typedef const __attribute__((address_space(4))) ResArgs* ConstArgs;
+__device__ __forceinline__ ConstArgs again(ConstArgs a) {
+  asm volatile("" : "+s"(a));
+  return a;
+}
+
+// The sum of v over the wave, in its last lane (row shifts and broadcasts of
+// the vector ALU: no LDS latency).
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_add(double v) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, ROWS, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, ROWS, 0xf, false);
+  return v + __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+__device__ __forceinline__ double wave_sum_last(double v) {
+  v = dpp_add<0x111, 0xf>(v);  // row_shr:1, 2, 4, 8
+  v = dpp_add<0x112, 0xf>(v);
+  v = dpp_add<0x114, 0xf>(v);
+  v = dpp_add<0x118, 0xf>(v);
+  v = dpp_add<0x142, 0xa>(v);  // row_bcast:15 into rows 1 and 3
+  return dpp_add<0x143, 0xc>(v);  // row_bcast:31 into rows 2 and 3
+}
+
+// The sum of v over the block, in thread 0, the waves' totals in wave order.
+__device__ __forceinline__ double res_block_sum(double v, int tid, int nthr, double* lds) {
+  for (int o = kWave / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, kWave);
+  if (tid % kWave == 0) lds[tid / kWave] = v;
+  __syncthreads();
+  double s = 0.0;
+  if (tid == 0)
+    for (int w = 0; w < nthr / kWave; w++) s += lds[w];
+  __syncthreads();
+  return s;
+}
+
+// Records iteration l's sum of reltmp^2 and returns whether it stops the
+// loop (press.f95:119-121, or a non-finite sum).
+__device__ __forceinline__ bool res_record(Ctrl* ctrl, int l, double s, float pjuge, bool writer) {
+  const bool bad = !(s == s) || s > 1.0e300;
+  const bool stop = s < (double)pjuge || bad;
+  if (writer) {
+    if (l <= kSorHist) ctrl->sor_hist[l - 1] = s;
+    ctrl->sor_iters = l;
+    if (bad) ctrl->nonfinite = 1;
+    if (stop) ctrl->sor_done = l;
+  }
+  return stop;
+}
+
+// The block after the boxes: the stop test of every iteration (press.f95:
+// 119-121), off the boxes' way.  Adds each iteration's partial sums in a fixed
+// order, records the total and publishes one word: its tag that of the sums,
+// its value 1 where the loop stops.
+__device__ __forceinline__ void res_monitor(ConstArgs a, int nb, unsigned tag, int tid, int nthr, double* lds) {
+  const int np = nb * (nthr / kWave);  // one partial sum per wave
+  for (int l = 1; l <= a->nmaxp; l++) {
+    const unsigned pt = tag + 2 * l;
+    double x = 0.0;
+    for (int b = tid; b < np; b += nthr) {
+      const u64* const pw = a->parts + ((size_t)(l & 3) * np + b) * 2;
+      u64 h = ald(pw), lo = ald(pw + 1);
+      for (int spin = 0; wtag(h) != pt || wtag(lo) != pt;) {
+        h = ald(pw);
+        lo = ald(pw + 1);
+        if (++spin > kSpinMax) return;  // cannot happen while every block runs
+      }
+      x += __longlong_as_double((long long)((h << 32) | (lo & 0xffffffffull)));
+    }
+    x = res_block_sum(x, tid, nthr, lds);
+    if (tid == 0) {
+      const bool stop = res_record(a->ctrl, l, x, a->pjuge, true);
+      ast(a->parts + 8 * (size_t)np + (l & 3), ((u64)pt << 32) | (stop ? 1u : 0u));
+      lds[0] = stop ? 1.0 : 0.0;
+    }
+    __syncthreads();
+    const bool stop = lds[0] != 0.0;
+    __syncthreads();
+    if (stop) return;
+  }
+}
+
+// Iteration l's word of the monitor: 1 where the loop stops.
+__device__ __forceinline__ int res_verdict(ConstArgs a, int np, int l, unsigned pt, int* dead) {
+  const u64* const pw = a->parts + 8 * (size_t)np + (l & 3);
+  u64 w = ald(pw);
+  for (int spin = 0; wtag(w) != pt;) {
+    w = ald(pw);
+    if (++spin > kSpinMax) {
+      *dead = 1;
+      break;
+    }
+  }
+  return (int)(w & 1u);
+}
+
+// 1: every block of the launch is resident; 2: they are not, and the launch
+// runs by tickets.  Thread 0 of each block; the last block to arrive decides
+// 1, a block that waited kEnterTicks (or force_ticket) decides 2, whichever
+// comes first.
+__device__ __forceinline__ int res_enter(Ctrl* ctrl, int nb, int force_ticket) {
+  if (force_ticket) return 2;
+  const int n = __hip_atomic_fetch_add(&ctrl->res_arrived, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (n == nb - 1) {
+    int want = 0;
+    __hip_atomic_compare_exchange_strong(&ctrl->res_state, &want, 1, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                         __HIP_MEMORY_SCOPE_AGENT);
+    return ald(&ctrl->res_state);
+  }
+  const long long t0 = wall_clock64();
+  for (;;) {
+    const int st = ald(&ctrl->res_state);
+    if (st != 0) return st;
+    if (wall_clock64() - t0 > kEnterTicks) {
+      int want = 0;
+      __hip_atomic_compare_exchange_strong(&ctrl->res_state, &want, 2, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                           __HIP_MEMORY_SCOPE_AGENT);
+      return ald(&ctrl->res_state);
+    }
+    __builtin_amdgcn_s_sleep(1);
+  }
+}
+
+// The solve without co-residency: colour sweeps over the split arrays (sets 0
+// and 1 by iteration parity, as k_sweep), each cut into tickets taken in
+// order.  A sweep starts when the one before is complete; its tickets were
+// taken before and are held by running blocks.
+__device__ __forceinline__ void res_ticket(ConstArgs a0, float* lds_f) {
+  double* const lds = (double*)lds_f;
+  int* const sh = (int*)(lds_f + 2 * (kResNT / kWave));
+  const int tid = threadIdx.x, nthr = blockDim.x;
+  const ConstArgs a = a0;
+  const Grid g = {a->g.im, a->g.jm, a->g.km, a->g.sj, a->g.sk};
+  const SplitGrid s = {a->s.nt, a->s.cp, a->s.cplane};
+  Ctrl* ctrl = a->ctrl;
+  const int im = g.im, jm = g.jm, km = g.km, nt = s.nt;
+  const int npr = nt * jm;                          // pairs per level
+  const int chunks = (npr + nthr - 1) / nthr;      // tickets per level
+  const int per = chunks * km;                      // tickets per sweep
+  for (;;) {
+    __syncthreads();
+    if (tid == 0)
+      sh[0] = __hip_atomic_fetch_add(&ctrl->tk_next, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    const int tk = sh[0];
+    // sweep 0 is the copy of the start iterate into set 0, sweep 2l-1 red of
+    // iteration l, 2l its black
+    const int sweep = tk / per, it = tk % per;
+    if (sweep > 2 * a->nmaxp) return;
+    if (tid == 0) {
+      sh[1] = 0;
+      for (int spin = 0; ald(&ctrl->tk_phase) < sweep; spin++) {
+        __builtin_amdgcn_s_sleep(2);
+        if (spin > kSpinMax) {  // cannot happen: the tickets waited for are held by running blocks
+          ctrl->nonfinite = 1;
+          sh[1] = 1;
+          break;
+        }
+      }
+      if (ald(&ctrl->sor_done) != 0) sh[1] = 1;
+    }
+    __syncthreads();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    if (sh[1] != 0) return;
+    const int l = (sweep + 1) / 2, col = sweep & 1;  // col 1 = red
+    const int src = (l - 1) & 1, dst = l & 1;
+    const int x = (it % chunks) * nthr + tid, k = 1 + it / chunks;
+    double acc = 0.0;
+    if (x < npr) {
+      const int t = x % nt, j = 1 + x / nt;
+      const int q = rcix(s, t, j, k);
+      if (sweep == 0) {
+        for (int c = 0; c < 2; c++) {
+          const int i = 2 * t + 1 + ((1 + j + k + c) & 1);
+          a->sb.p[0][c][q] = (a->zero || i > im) ? 0.0f : a->pent[ix(g, i, j, k)];
+        }
+      } else {
+        const int pos = (1 + j + k + col) & 1, i = 2 * t + 1 + pos;
+        if (i <= im) {
+          const float* own_ = a->sb.p[src][col];
+          const float* oth = a->sb.p[col ? src : dst][col ^ 1];
+          const float own = own_[q];
+          const bool ent = l == 1 && !a->zero;  // iteration 1 reads the ghosts p had on entry
+          // i ghosts mirror the cell; j wraps (the cell's own colour when jm is odd); k ghosts mirror
+          float lo = (i == 1) ? own : oth[q - 1 + pos];
+          float hi = (i == im) ? own : oth[q + pos];
+          const float* wr = (jm & 1) ? own_ : oth;
+          float pjm = (j == 1) ? wr[rcix(s, t, jm, k)] : oth[q - s.cp];
+          float pjp = (j == jm) ? wr[rcix(s, t, 1, k)] : oth[q + s.cp];
+          float pkm = (k == 1) ? own : oth[q - s.cplane];
+          float pkp = (k == km) ? own : oth[q + s.cplane];
+          if (ent) {
+            if (col == 1) {
+              if (i == 1) lo = a->pent[ix(g, 0, j, k)];
+              if (i == im) hi = a->pent[ix(g, im + 1, j, k)];
+              if (j == 1) pjm = a->pent[ix(g, i, 0, k)];
+              if (j == jm) pjp = a->pent[ix(g, i, jm + 1, k)];
+            }
+            if (k == 1) pkm = a->pent[ix(g, i, j, 0)];
+            if (k == km) pkp = a->pent[ix(g, i, j, km + 1)];
+          }
+          const float rel = a->omega * (a->m.lev4[4 * k + 2] * (a->c2 * hi + a->c2 * lo + a->c3 * pjp + a->c3 * pjm +
+                                                          M1(a->m.cn4l, k) * pkp + M1(a->m.cn4s, k) * pkm -
+                                                          a->sb.rhs[col][q]) -
+                                       own);
+          a->sb.p[dst][col][q] = own + rel;
+          acc = (double)rel * (double)rel;
+        }
+      }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+    const double bsum = res_block_sum(acc, tid, nthr, lds);  // its barriers: every store of the block is released
+    if (tid == 0) {
+      ast((u64*)&a->tparts[(size_t)(sweep & 3) * per + it], (u64)__double_as_longlong(bsum));
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+      sh[0] = __hip_atomic_fetch_add(&ctrl->tk_done, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    }
+    __syncthreads();
+    if (sh[0] != (sweep + 1) * per - 1) continue;
+    // the sweep's last ticket: iteration l's sum after its black sweep, then the next sweep
+    double tot = 0.0;
+    if (sweep > 0 && col == 0) {
+      for (int b = tid; b < per; b += nthr) {
+        tot += __longlong_as_double((long long)ald((u64*)&a->tparts[(size_t)((sweep - 1) & 3) * per + b]));
+        tot += __longlong_as_double((long long)ald((u64*)&a->tparts[(size_t)(sweep & 3) * per + b]));
+      }
+      tot = res_block_sum(tot, tid, nthr, lds);
+    }
+    if (tid == 0) {
+      bool stop = false;
+      if (sweep > 0 && col == 0) {
+        stop = res_record(ctrl, l, tot, a->pjuge, true);
+        ctrl->p_final = l & 1;
+      }
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+      // a stop ends every wait: the tickets of later sweeps find sor_done
+      ast(&ctrl->tk_phase, stop ? 0x7fffffff : sweep + 1);
+    }
+  }
+}
+
+// The resident solve of one box.  CLS: the kernel (kResClass); a block is
+// launched with as many waves as its largest box has columns or halo words
+// for.  BK: the most levels of a box, of which a box has BK-4 to BK.  OM1:
+// omega == 1 (1*y is y: the multiplication is dropped).  ODD: im is odd, so
+// the last pair of a row has one cell.
+template <int CLS, int BK, bool OM1, bool ODD>
+__device__ __forceinline__ void res_block(ConstArgs a0, const int bid) {
+  constexpr int PLANE = kResClass[CLS].plane, NW = kResClass[CLS].words, G = kResClass[CLS].group;
+  constexpr int NG = (BK + G - 1) / G, NT = kResNT, RL = res_lds_rhs(CLS, BK);
+  __shared__ float S[BK * PLANE];
+  __shared__ float RB[RL > 0 ? RL * NT : 1];  // rhs of the black cells of levels below RL, by thread
+  __shared__ double wsum[NT / kWave];
+  __shared__ int sh[3];  // mode; a wait that gave up; the monitor's verdict
+  const int tid = threadIdx.x, nthr = blockDim.x, nwav = nthr / kWave;
+  const int nb = a0->nb;
+  if (tid == 0) {
+    // sor_done set on entry (a finished defect correction): nothing to solve
+    sh[0] = a0->ctrl->sor_done != 0 ? 0 : res_enter(a0->ctrl, nb + 1, a0->force_ticket);
+    sh[1] = 0;
+  }
+  __syncthreads();
+  const int mode = sh[0];
+  if (mode == 0) return;
+  if (mode == 2) {
+    res_ticket(a0, S);
+    return;
+  }
+  if (bid == nb) {
+    res_monitor(again(a0), nb, (unsigned)a0->ctrl->res_epoch * 8192u, tid, nthr, wsum);
+    return;
+  }
+  const int W = a0->tp + 2;  // LDS row pitch; halo columns 0 and tpn+1, halo rows 0 and tjn+1
+  const bool oddj = (a0->g.jm & 1) != 0;
+  // balanced cuts: box sizes differ by at most one in each direction
+  const int bx = bid % a0->ntx, by = (bid / a0->ntx) % a0->nty, bz = bid / (a0->ntx * a0->nty);
+  const int k0 = 1 + bz * a0->g.km / a0->ntz, nlev = (bz + 1) * a0->g.km / a0->ntz + 1 - k0;
+  const bool kbot = bz == 0, ktop = bz == a0->ntz - 1;
+  int cent, side, rowd = 0;
+  bool act, wl[2], inv[2], wrl, wrh;
+  unsigned wsd[NW], wto[NW];  // S source | S destination; word in the inboxes | destination by colour << 31
+  {
+    const ConstArgs a = again(a0);
+    const int nt = a->s.nt, jm = a->g.jm, im = a->g.im;
+    const int t0 = bx * nt / a->ntx, tpn = (bx + 1) * nt / a->ntx - t0;
+    const int j0 = 1 + by * jm / a->nty, tjn = (by + 1) * jm / a->nty + 1 - j0;
+    const int row = tid / tpn, t = tid % tpn;
+    act = row < tjn;
+    const int tg = t0 + t;
+    const int par = (j0 + row + k0) & 1;  // position (i = 2t+1+position) of the red cell at the first level
+    const bool wlo = tg == 0, whi = tg == nt - 1;
+    // a cell at position 0 has its other in-row neighbour in pair t-1, at
+    // position 1 in pair t+1; red of level kk takes side kk & 1, black the
+    // other.  Threads without a column read cell 0 and write nothing.
+    cent = act ? (row + 1) * W + t + 1 : W + 1;
+    side = par ? 1 : -1;
+    wl[0] = par ? whi : wlo;  // the side lies beyond a wall
+    wl[1] = par ? wlo : whi;
+    const bool lastp = ODD && whi && (im & 1);  // the pair with one cell (position 0)
+    inv[0] = lastp && par == 1;                 // the cell using that side does not exist
+    inv[1] = lastp && par == 0;
+    // odd jm: across the periodic boundary the neighbour has the cell's own
+    // colour and keeps its previous iterate: rows tj+2 + 2c + side hold it
+    wrl = oddj && by == 0 && row == 0;
+    wrh = oddj && by == a->nty - 1 && row == tjn - 1;
+    rowd = (a->tj + 1 - row) * W;
+    // in-plane halo words e = tid + q*nthr, sent after every sweep of either
+    // colour: ranges i-lo, i-hi (row, level), j-lo, j-hi (level, pair).  A box
+    // sends word e to the next box up (lo) or down (hi) the direction, whose
+    // halo its range is, and receives its own word e.  No branch on what a
+    // word holds: the boxes form a ring in i too, where the word that crosses
+    // the walls goes to the last cell of the plane, as the words of rows,
+    // pairs or levels a box does not have; a face of which only the other
+    // colour has cells in a row is sent as well, into a halo cell not read then.
+    const int kl = a->kl, NI = a->ntx > 1 ? a->tj * kl : 0, NJ = a->tp * kl, IW = a->iw;
+#pragma unroll
+    for (int q = 0; q < NW; q++) {
+      const int e = tid + q * nthr;
+      unsigned so = 0, de = PLANE - 1, wrap = 0;
+      int to = bid;
+      if (e < 2 * NI) {
+        const int hi = e >= NI, x = hi ? e - NI : e, r = x / kl, kk = x % kl;
+        to = bid - bx + (hi ? bx + a->ntx - 1 : bx + 1) % a->ntx;
+        if (r < tjn && kk < nlev) {
+          so = kk * PLANE + (r + 1) * W + (hi ? 1 : tpn);
+          if (hi ? bx < a->ntx - 1 : bx > 0) de = kk * PLANE + (r + 1) * W + (hi ? tpn + 1 : 0);
+        }
+      } else if (e < 2 * NI + 2 * NJ) {
+        const int f = e - 2 * NI, hi = f >= NJ, x = hi ? f - NJ : f, kk = x / a->tp, p = x % a->tp;
+        to = bx + a->ntx * ((hi ? by + a->nty - 1 : by + 1) % a->nty + a->nty * bz);
+        if (p < tpn && kk < nlev) {
+          so = kk * PLANE + (hi ? 1 : tjn) * W + p + 1;
+          wrap = oddj && (hi ? by == a->nty - 1 : by == 0);  // kept by colour
+          de = kk * PLANE + (wrap ? a->tj + 2 + hi : hi ? tjn + 1 : 0) * W + p + 1;
+        }
+      }
+      wsd[q] = so | (de << 16);
+      wto[q] = (unsigned)(to * IW + e) | (wrap << 31);
+    }
+  }
+  const int nq = a0->nq;                    // halo words per thread
+  const unsigned nw0 = (unsigned)(nq * nthr);  // the k words follow the in-plane ones
+  const unsigned tag0 = (unsigned)a0->ctrl->res_epoch * 8192u;
+  const bool writer = bid == 0 && tid == 0;
+  float v[2][BK], rh[2][BK];  // [0] black, [1] red: iterate and rhs by level
+  float hlo[2], hhi[2];       // the k neighbours of colour c outside the box
+  int limit = a0->nmaxp;
+  bool dead = false;
+  const float c2 = a0->c2, c3 = a0->c3, omega = a0->omega;
+  // per level: cn4l, cn4s, cn1; those of the first group are kept
+  const ConstF lv0 = constf(a0->m.lev4 + 4 * k0);
+  float cu0[G], cl0[G], cn0[G];
+#pragma unroll
+  for (int u = 0; u < G; u++) {
+    cu0[u] = lv0[4 * u];
+    cl0[u] = lv0[4 * u + 1];
+    cn0[u] = lv0[4 * u + 2];
+  }
+  const bool zero0 = a0->zero != 0;
+
+  for (int pass = 0; pass < 2; pass++) {
+    const unsigned tag = tag0 + pass * 4096u;
+    __syncthreads();
+    // ---- the start iterate and its halo (the padded field holds the ghosts
+    // p had on entry, which iteration 1 reads)
+    {
+      const ConstArgs a = again(a0);
+      int ce = cent;
+      asm volatile("" : "+v"(ce));  // addresses made here, not held over the solve
+      const Grid g = {a->g.im, a->g.jm, a->g.km, a->g.sj, a->g.sk};
+      const SplitGrid s = {a->s.nt, a->s.cp, a->s.cplane};
+      const float* const pent = a->pent;
+      const bool zero = a->zero != 0;
+      const int t0 = bx * s.nt / a->ntx, tpn = (bx + 1) * s.nt / a->ntx - t0;
+      const int j0 = 1 + by * g.jm / a->nty, tjn = (by + 1) * g.jm / a->nty + 1 - j0;
+      const int tg = t0 + ce % W - 1, j = j0 + ce / W - 1;
+      {
+        const float* r0 = a->sb.rhs[0] + rcix(s, tg, j, k0);
+        const float* r1 = a->sb.rhs[1] + rcix(s, tg, j, k0);
+        const float* pp = pent + ix(g, 2 * tg + 1, j, k0);  // i = 1 is 256-byte aligned
+#pragma unroll
+        for (int kk = 0; kk < BK; kk++) {
+          v[0][kk] = v[1][kk] = rh[0][kk] = rh[1][kk] = 0.0f;
+          if (kk < BK - 4 || kk < nlev) {
+            if (kk < RL)
+              RB[kk * NT + tid] = *r0;
+            else
+              rh[0][kk] = *r0;
+            rh[1][kk] = *r1;
+            if (!zero) {
+              const float2 x = *(const float2*)pp;
+              const bool pr = (side > 0) != ((kk & 1) != 0);  // red at position 1
+              v[1][kk] = pr ? x.y : x.x;
+              v[0][kk] = pr ? x.x : x.y;
+            }
+            r0 += s.cplane;
+            r1 += s.cplane;
+            pp += g.sk;
+          }
+        }
+      }
+      for (int c = 0; c < 2; c++) hlo[c] = hhi[c] = 0.0f;
+      if (!zero) {
+        for (int c = 0; c < 2; c++) {  // colour c at level k sits where the other colour does at k -+ 1
+          hlo[c] = pent[ix(g, 2 * tg + 1 + ((1 + j + k0 + c) & 1), j, k0 - 1)];
+          const int k1 = k0 + nlev - 1;
+          hhi[c] = pent[ix(g, 2 * tg + 1 + ((1 + j + k1 + c) & 1), j, k1 + 1)];
+        }
+      }
+      // the black cells and the in-plane halo the first red sweep reads
+      if (act) {
+#pragma unroll
+        for (int kk = 0; kk < BK; kk++)
+          if (kk < BK - 4 || kk < nlev) S[kk * PLANE + ce] = v[0][kk];
+      }
+      for (int x = tid; x < (tpn + tjn) * 2 * nlev; x += nthr) {
+        const int kk = x / (2 * (tpn + tjn)), y = x % (2 * (tpn + tjn)), k = k0 + kk;
+        if (y < 2 * tpn) {
+          const int hi = y >= tpn, p = hi ? y - tpn : y, tt = t0 + p;
+          const int je = hi ? j0 + tjn - 1 : j0, jn = hi ? je + 1 : je - 1;  // edge row and the row beyond
+          const int i = 2 * tt + 1 + ((1 + je + k + 1) & 1);                 // red of the edge row
+          const float x0 = zero ? 0.0f : pent[ix(g, i, jn, k)];
+          if (oddj && (hi ? je == g.jm : je == 1)) {
+            S[kk * PLANE + (a->tj + 4 + hi) * W + p + 1] = x0;  // red
+            const int ib = 2 * tt + 1 + ((1 + je + k) & 1);     // black of the edge row: the wrapped row itself
+            S[kk * PLANE + (a->tj + 2 + hi) * W + p + 1] =
+                (zero || ib > g.im) ? 0.0f : pent[ix(g, ib, hi ? 1 : g.jm, k)];
+          } else {
+            S[kk * PLANE + (hi ? tjn + 1 : 0) * W + p + 1] = x0;
+          }
+        } else {
+          const int z = y - 2 * tpn, hi = z >= tjn, r = hi ? z - tjn : z;
+          const int i = hi ? 2 * (t0 + tpn) + 1 : 2 * t0;
+          S[kk * PLANE + (r + 1) * W + (hi ? tpn + 1 : 0)] = zero ? 0.0f : pent[ix(g, i, j0 + r, k)];
+        }
+      }
+    }
+    __syncthreads();
+
+    int stop_at = 0;
+    for (int l = 1; l <= limit; l++) {
+      double acc = 0.0;
+#pragma unroll
+      for (int cc = 1; cc >= 0; cc--) {
+        const int c = cc;  // 1 red, 0 black
+        const unsigned wt = tag + 2 * l + c;
+        const bool later = l > 1 || zero0;  // walls mirror (a zero start has zero ghosts either way)
+        // ---- the colour sweep
+        {
+          float below_v = hlo[c];
+          if (kbot && later) below_v = v[c][0];
+          const bool mir = later || c == 0;
+          const bool wall0 = wl[c ^ 1] && mir, wall1 = wl[c] && mir;
+          const bool own_top = ktop && later;
+          // the LDS address of every access is an immediate offset from these
+          // four (as loop invariants the compiler would hold one per access)
+          asm volatile("" : "+v"(cent));
+          const int al[2] = {cent + side, cent - side};
+          int au = cent - W, ad = cent + W;
+          if (oddj) {
+            const int xr = cent + rowd + 2 * c * W;
+            au = wrl ? xr : au;
+            ad = wrh ? xr + W : ad;
+          }
+          int tr = tid;
+          asm volatile("" : "+v"(tr));
+          ConstF lv = lv0;
+          asm volatile("" : "+s"(lv));
+          // groups of G levels; a group's operands are fetched while the one
+          // before is computed
+          float lat[2][G], pjm[2][G], pjp[2][G], rb[2][G], cu[2][G], cl[2][G], cn[2][G];
+          auto fetch = [&](auto gi) {
+            constexpr int g0 = decltype(gi)::value, b = g0 & 1;
+#pragma unroll
+            for (int u = 0; u < G; u++) {
+              const int kk = g0 * G + u;
+              if (kk < BK) {
+                const float* P = S + kk * PLANE;
+                lat[b][u] = P[al[(kk & 1) ^ (c ^ 1)]];
+                pjm[b][u] = P[au];
+                pjp[b][u] = P[ad];
+                rb[b][u] = (c == 0 && kk < RL) ? RB[kk * NT + tr] : rh[c][kk];
+                cu[b][u] = g0 == 0 ? cu0[u] : lv[4 * kk];
+                cl[b][u] = g0 == 0 ? cl0[u] : lv[4 * kk + 1];
+                cn[b][u] = g0 == 0 ? cn0[u] : lv[4 * kk + 2];
+              }
+            }
+          };
+          auto ready = [&](auto gi) {  // wait for the group here, before the next one's loads are issued
+            constexpr int g0 = decltype(gi)::value, b = g0 & 1;
+#pragma unroll
+            for (int u = 0; u < G; u++)
+              if (g0 * G + u < BK) {
+                const float x0 = lat[b][u], x1 = pjm[b][u], x2 = pjp[b][u], x3 = rb[b][u], y0 = cu[b][u], y1 = cl[b][u], y2 = cn[b][u];
+                asm volatile("" ::"v"(x0), "v"(x1), "v"(x2), "v"(x3), "s"(y0), "s"(y1), "s"(y2));
+              }
+          };
+          auto compute = [&](auto gi) {
+            constexpr int g0 = decltype(gi)::value, b = g0 & 1;
+#pragma unroll
+            for (int u = 0; u < G; u++) {
+              const int kk = g0 * G + u;
+              if (kk < BK && (kk < BK - 4 || kk < nlev)) {
+                const int ai = (kk & 1) ^ (c ^ 1);
+                const float own = v[c][kk];
+                float oth = v[c ^ 1][kk];
+                const float la = ((kk & 1) ? wall1 : wall0) ? own : lat[b][u];
+                if (ODD) oth = (inv[ai ^ 1] && mir) ? own : oth;  // the pair's other cell is the ghost at im+1
+                const float pkm = kk == 0 ? below_v : v[c ^ 1][kk > 0 ? kk - 1 : 0];
+                float pkp = v[c ^ 1][kk < BK - 1 ? kk + 1 : kk];
+                if (kk >= BK - 5) {
+                  if (kk == nlev - 1) pkp = own_top ? own : hhi[c];
+                }
+                const float x = c2 * la + c2 * oth + c3 * pjp[b][u] + c3 * pjm[b][u] + cu[b][u] * pkp +
+                                cl[b][u] * pkm - rb[b][u];
+                float rel = cn[b][u] * x - own;
+                if (!OM1) rel = omega * rel;
+                if (ODD) rel = inv[ai] ? 0.0f : rel;
+                acc = __builtin_fma((double)rel, (double)rel, acc);
+                v[c][kk] = own + rel;
+              }
+            }
+          };
+          auto run = [&](auto self, auto gi) {
+            constexpr int g0 = decltype(gi)::value;
+            if constexpr (g0 < NG) {
+              ready(gi);
+              if constexpr (g0 + 1 < NG) fetch(std::integral_constant<int, g0 + 1>{});
+              __builtin_amdgcn_sched_barrier(0);
+              compute(gi);
+              __builtin_amdgcn_sched_barrier(0);
+              self(self, std::integral_constant<int, g0 + 1>{});
+            }
+          };
+          fetch(std::integral_constant<int, 0>{});
+          run(run, std::integral_constant<int, 0>{});
+        }
+        const ConstArgs a = again(a0);
+        u64* const inb = a->slots + (c ? (unsigned)nb * (unsigned)a->iw : 0u);  // red inboxes after the black ones
+        // (nothing derived from these is to be held over the loop)
+        unsigned tx = tid;
+        int nl = nlev, nqo = nq;
+        asm volatile("" : "+v"(tx), "+s"(nl), "+s"(nqo));
+#pragma unroll
+        for (int q = 0; q < NW; q++) asm volatile("" : "+v"(wsd[q]), "+v"(wto[q]));
+        // the k faces: my first level is the box below's k-hi, my last the
+        // box above's k-lo (the same columns, so the same threads, without
+        // one the same too)
+        if (!kbot) ast(inb + (unsigned)((bid - a->ntx * a->nty) * a->iw) + nw0 + NT + tx, word(wt, v[c][0]));
+        if (!ktop) {
+          float vtop = v[c][BK - 1];
+#pragma unroll
+          for (int kk = BK > 5 ? BK - 5 : 0; kk < BK - 1; kk++) vtop = kk == nl - 1 ? v[c][kk] : vtop;
+          ast(inb + (unsigned)((bid + a->ntx * a->nty) * a->iw) + nw0 + tx, word(wt, vtop));
+        }
+        __syncthreads();  // every read of the other colour's copy is done
+        if (act) {
+#pragma unroll
+          for (int kk = 0; kk < BK; kk++) S[kk * PLANE + cent] = v[c][kk];  // levels from nlev on are not read
+        }
+        __syncthreads();  // the copy holds colour c
+        // ---- send the in-plane faces
+        const int cw = 2 * c * W;
+        if (nb == 1) {  // a box that is its own neighbour
+#pragma unroll
+          for (int q = 0; q < NW; q++)
+            if (q < nqo) S[(wsd[q] >> 16) + ((wto[q] >> 31) ? cw : 0)] = S[wsd[q] & 0xffffu];
+        } else {
+          float x[NW];
+#pragma unroll
+          for (int q = 0; q < NW; q++)
+            if (q < nqo) x[q] = S[wsd[q] & 0xffffu];
+#pragma unroll
+          for (int q = 0; q < NW; q++)
+            if (q < nqo) ast(inb + (wto[q] & 0x7fffffffu), word(wt, x[q]));
+        }
+        if (c == 0 && pass == 0) {  // the iteration's sum of reltmp^2, wave by wave (while the words cross)
+          const double x = wave_sum_last(act ? acc : 0.0);
+          if (tid % kWave == kWave - 1) {
+            const u64 bits = (u64)__double_as_longlong(x), wq = (u64)wt << 32;
+            u64* const pw = a->parts + ((size_t)(l & 3) * (nb * nwav) + (bid * nwav + tid / kWave)) * 2;
+            ast(pw, wq | (bits >> 32));
+            ast(pw + 1, wq | (bits & 0xffffffffull));
+          }
+        }
+        // ---- receive the halo
+        if (nb > 1) {
+          const u64* const me = inb + (unsigned)(bid * a->iw);
+          u64 w[NW], wk[2] = {0, 0};
+          for (int spin = 0;; spin++) {
+            unsigned miss = 0;
+            if (!kbot) wk[0] = ald(me + nw0 + tx);
+            if (!ktop) wk[1] = ald(me + nw0 + NT + tx);
+#pragma unroll
+            for (int q = 0; q < NW; q++)
+              if (q < nqo) w[q] = ald(me + tx + q * nthr);
+            if (!kbot) miss |= wtag(wk[0]) ^ wt;
+            if (!ktop) miss |= wtag(wk[1]) ^ wt;
+#pragma unroll
+            for (int q = 0; q < NW; q++)
+              if (q < nqo) miss |= wtag(w[q]) ^ wt;
+            if (miss == 0) break;
+            if (spin > kSpinMax) {  // cannot happen while every block runs
+              sh[1] = 1;
+              break;
+            }
+          }
+          if (!kbot) hlo[c ^ 1] = wval(wk[0]);
+          if (!ktop) hhi[c ^ 1] = wval(wk[1]);
+#pragma unroll
+          for (int q = 0; q < NW; q++)
+            if (q < nqo) S[(wsd[q] >> 16) + ((wto[q] >> 31) ? cw : 0)] = wval(w[q]);
+        }
+        {
+          // the verdict on iteration l-2, published during l-1
+          if (c == 0 && pass == 0 && l > 2 && tid == 0)
+            sh[2] = res_verdict(a, nb * nwav, l - 2, tag + 2 * (l - 2), &sh[1]);
+        }
+        __syncthreads();  // the halo is in place
+        if (sh[1]) {
+          dead = true;
+          break;
+        }
+      }
+      if (dead) break;
+      if (pass == 0 && l > 2 && sh[2]) {
+        stop_at = l - 2;
+        break;
+      }
+    }
+    if (dead) {
+      if (tid == 0) a0->ctrl->nonfinite = 1;
+      break;
+    }
+    if (pass == 1) break;
+    if (stop_at == 0) {  // the verdicts not yet seen
+      __syncthreads();
+      if (tid == 0) {
+        const ConstArgs a = again(a0);
+        int at = 0;
+        for (int l = max(1, limit - 1); l <= limit && at == 0; l++)
+          if (res_verdict(a, nb * nwav, l, tag + 2 * l, &sh[1])) at = l;
+        sh[2] = at;
+      }
+      __syncthreads();
+      stop_at = sh[2];
+      if (stop_at == 0 || stop_at == limit) break;  // the registers hold iterate `limit`
+    }
+    // the loop ran past the iteration that stopped it: run again from the
+    // start, which the solve has not changed, to exactly that one
+    limit = stop_at;
+  }
+  {
+    const ConstArgs a = again(a0);
+    const int t0 = bx * a->s.nt / a->ntx, j0 = 1 + by * a->g.jm / a->nty;
+    const int q0 = rcix({a->s.nt, a->s.cp, a->s.cplane}, t0 + cent % W - 1, j0 + cent / W - 1, k0), cpl = a->s.cplane;
+    float* const b = a->sb.p[1][0] + q0;
+    float* const r = a->sb.p[1][1] + q0;
+    if (act) {
+#pragma unroll
+      for (int kk = 0; kk < BK; kk++)
+        if (kk < BK - 4 || kk < nlev) {
+          b[kk * cpl] = v[0][kk];
+          r[kk * cpl] = v[1][kk];
+        }
+    }
+    if (writer) a->ctrl->p_final = 1;
+  }
+}
+
+template <int CLS, int BK, bool OM1, bool ODD>
+__global__ __launch_bounds__(kResNT, 2 * kResClass[CLS].per) void k_sor_res(ResArgs a) {
+  (void)a;  // the kernel argument segment starts with it
+  res_block<CLS, BK, OM1, ODD>((ConstArgs)__builtin_amdgcn_kernarg_segment_ptr(), (int)blockIdx.x);
+}
+
+}  // namespace
+
+// Microseconds of one sweep of a cut, as a model: the sweep of a unit's boxes
+// (80 cycles per level and wave of a SIMD, no less than the latency of a wave
+// alone), the exchange (latency, and words per unit), and what a box of two
+// hides of it.
+static double res_cost(int waves, int kl, int nb, int words, int cls, int units) {
+  const int on = nb > units ? 2 : 1;  // boxes on the fullest unit
+  const double sweep = std::max(0.034 * ((on * waves + 3) / 4), 0.055) * kl + 0.3 + 0.05 * waves * on;
+  const double cross = nb > 1 ? 1.5 + 0.35 * on * words / 1024 : 0.0;
+  (void)cls;
+  return on == 1 ? sweep + cross : std::max(sweep, 0.6 * sweep + cross);
+}
+
+// The cut of a domain into boxes with the least modelled time.  False when
+// no cut fits (about 12 million cells on 256 units).
+bool res_shape(const Grid& g, const SplitGrid& s, int units, ResShape* out) {
+  double best = -1.0;
+  const auto up = [](int a, int b) { return (a + b - 1) / b; };
+  for (int cls = 0; cls < 2; cls++) {
+    const ResClass C = kResClass[cls];
+    const int nmax = C.per * units - 1;  // one block runs the monitor
+    for (int ntz = 1; ntz <= std::min(g.km, nmax); ntz++) {
+      const int kl = up(g.km, ntz);
+      if (kl > C.levels || (ntz > 1 && kl == up(g.km, ntz - 1))) continue;
+      for (int ntx = 1; ntx <= s.nt && ntx * ntz <= nmax; ntx++) {
+        const int tp = up(s.nt, ntx);
+        if (tp > kResNT || (ntx > 1 && tp == up(s.nt, ntx - 1))) continue;
+        for (int nty = std::max(1, up(g.jm, kResNT / tp)); nty <= g.jm && ntx * nty * ntz <= nmax; nty++) {
+          const int tj = up(g.jm, nty);
+          if (tp * tj > kResNT || (nty > 1 && tj == up(g.jm, nty - 1))) continue;
+          if ((tp + 2) * (tj + 2 + ((g.jm & 1) ? 4 : 0)) >= C.plane) continue;
+          const int ni = ntx > 1 ? tj * kl : 0, nj = tp * kl, nb = ntx * nty * ntz, wds = 2 * ni + 2 * nj;
+          // whole waves, enough for the columns and for the halo words
+          const int nthr = up(std::max(tp * tj, up(wds, C.words)), kWave) * kWave;
+          if (nthr > kResNT) continue;
+          const int nq = up(wds, nthr);
+          const double cost = res_cost(nthr / kWave, kl, nb, wds + (ntz > 1 ? 2 * nthr : 0), cls, units);
+          if (best < 0.0 || cost < best) {
+            best = cost;
+            *out = ResShape{ntx, nty, ntz, tp, tj, kl, nb, nq * nthr + 2 * kResNT, nq, cls, nthr};
+          }
+        }
+      }
+    }
+  }
+  return best >= 0.0;
+}
+
+// 8-byte words of the workspace: inboxes of both colours, the partial sums
+// of four iterations (two words each) and their verdicts, and the partial sums of the ticket
+// sweeps.
+static long res_tickets(const Grid& g, const SplitGrid& s) {
+  return (long)((s.nt * (long)g.jm + 63) / 64) * g.km;  // blocks of at least 64 threads
+}
+long res_words(const Grid& g, const SplitGrid& s, const ResShape& h) {
+  return 2L * h.nb * h.iw + 8L * h.nb * (h.nthr / kWave) + 8 + 4 * res_tickets(g, s);
+}
+
+template <int CLS, bool OM1, bool ODD>
+static void launch_res(const DevDomain& d, const ResArgs& a) {
+  const dim3 grid(d.res.nb + 1), blk(d.res.nthr);
+#define RES(BK)                                                                                          \
+  if (d.res.kl <= BK) {                                                                                  \
+    TIMED(d, KC_SOR, hipLaunchKernelGGL((k_sor_res<CLS, BK, OM1, ODD>), grid, blk, 0, d.stream, a));      \
+    return;                                                                                              \
+  }
+  RES(4)
+  RES(8)
+  RES(12)
+  RES(16)
+  RES(20)
+  RES(24)
+  if constexpr (CLS == 0) {
+    RES(28)
+    RES(32)
+    RES(36)
+    RES(40)
+  }
+#undef RES
+}
+
+void launch_sor_res(const DevDomain& d, const SplitBufs& sb, int nmaxp, float pjuge, float omega, bool zero) {
+  const ResShape& h = d.res;
+  ResArgs a{};
+  a.g = d.g;
+  a.s = d.sg;
+  a.m = d.m;
+  a.sb = sb;
+  a.ctrl = d.ctrl;
+  a.pent = d.F.p;
+  a.slots = d.res_mem;
+  a.parts = d.res_mem + 2L * h.nb * h.iw;
+  a.tparts = (double*)(a.parts + 8L * h.nb * (h.nthr / kWave) + 8);
+  a.c2 = d.res_c2;
+  a.c3 = d.res_c3;
+  a.omega = omega;
+  a.pjuge = pjuge;
+  a.nmaxp = nmaxp;
+  a.zero = zero;
+  a.force_ticket = d.res_on == 2;
+  a.ntx = h.ntx;
+  a.nty = h.nty;
+  a.ntz = h.ntz;
+  a.tp = h.tp;
+  a.tj = h.tj;
+  a.kl = h.kl;
+  a.nb = h.nb;
+  a.iw = h.iw;
+  a.nq = h.nq;
+  const bool odd = (d.g.im & 1) != 0;
+  if (h.cls == 0) {
+    if (omega != 1.0f)
+      launch_res<0, false, true>(d, a);
+    else if (odd)
+      launch_res<0, true, true>(d, a);
+    else
+      launch_res<0, true, false>(d, a);
+  } else {
+    if (omega != 1.0f)
+      launch_res<1, false, true>(d, a);
+    else if (odd)
+      launch_res<1, true, true>(d, a);
+    else
+      launch_res<1, true, false>(d, a);
+  }
+}
+
+}  // namespace les

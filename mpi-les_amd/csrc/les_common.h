@@ -49,6 +49,7 @@ struct Metrics {
   const float* cnax;    // 2/(dxs(i-1)*dxs(i)), the three terms of cn1 (init.f95:100-107)
   const float* cnby;    // 2/(dys(j-1)*dys(j))
   const float* cncz;    // 2/(dzs(k-1)*dzs(k))
+  const float* lev4;    // four floats per level from 4k: cn4l, cn4s, and cn1 = 1/((cnax+cnby)+cncz(k)) where those are uniform
   const float* inflow;    // u_in(j,k) at (j-1)+(k-1)*jm, nullptr = 5 m/s
   const float* inflow_v;  // v_in(j,k), nullptr = 0 (bondv1_data24.f95:79-87 reads all three)
   const float* inflow_w;  // w_in(j,k), nullptr = 0
@@ -72,6 +73,10 @@ struct Ctrl {
   int fix_in, fix_out;     // ... from iterate set fix_in into set fix_out
   int dc_done;             // press mode 1: the defect met the stop threshold (later outer steps skip)
   int dc_norms;            // press mode 1: defect norms recorded in this press call
+  // the one-launch SOR (k_sor_res), set up by the kernel before it: number of
+  // the solve (the words of earlier ones are told by it), blocks that have
+  // entered, 1 all resident / 2 by tickets, and the ticket counters
+  int res_epoch, res_arrived, res_state, tk_next, tk_phase, tk_done;
   double rhsav;            // volume-weighted mean of rhs
   double pav;              // volume-weighted mean of p
   double sor_first;        // sum of reltmp^2 of the current iteration's first colour
@@ -80,6 +85,13 @@ struct Ctrl {
 };
 
 constexpr int kWave = 64;
+
+// Before a launch of k_sor_res, in one thread of an earlier kernel.
+__device__ __forceinline__ void res_begin(Ctrl* ctrl) {
+  ctrl->res_epoch++;
+  ctrl->res_arrived = ctrl->res_state = 0;
+  ctrl->tk_next = ctrl->tk_phase = ctrl->tk_done = 0;
+}
 
 // The row of a block whose rows are one wave wide (blockDim.x == 64): the
 // same for every lane of a wave, so the compiler can keep it, and whatever

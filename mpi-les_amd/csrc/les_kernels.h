@@ -39,6 +39,30 @@ struct SplitBufs {
   int nplanes;          // planes in the allocation (10 km + 2)
 };
 
+// The cut of a domain into the boxes of the one-launch SOR (k_sor_res).
+struct ResShape {
+  int ntx, nty, ntz;  // boxes along the pairs, the rows and the levels
+  int tp, tj, kl;     // pairs, rows and levels of the largest box
+  int nb;             // boxes, one block each
+  int iw;             // halo words of one box's inbox, per colour
+  int nq;             // in-plane halo words per thread
+  int cls, nthr;      // the kernel (one block per compute unit, or two) and the threads launched
+};
+struct ResArgs {
+  Grid g;
+  SplitGrid s;
+  Metrics m;
+  SplitBufs sb;                // reads rhs, writes iterate set 1
+  Ctrl* ctrl;
+  const float* pent;           // the padded field p: start iterate and the ghosts it had on entry
+  unsigned long long* slots;   // halo words: inboxes of the black, then of the red cells
+  unsigned long long* parts;   // partial sums of four iterations, two words each
+  double* tparts;              // partial sums of the ticket sweeps
+  float c2, c3, omega, pjuge;  // uniform cn2l = cn2s, cn3l = cn3s
+  int nmaxp, zero, force_ticket;  // zero: start from p = 0 instead of pent
+  int ntx, nty, ntz, tp, tj, kl, nb, iw, nq;
+};
+
 // Kernel classes for the optional per-launch timing (les_domain_set_timing).
 enum KClass {
   KC_VELNW, KC_BONDV1, KC_VEL2, KC_VEL2_GHOST, KC_VELFG, KC_FEEDBF, KC_LES_SM, KC_BOUNDSM,
@@ -91,8 +115,21 @@ struct DevDomain {
   // height map zbm for masks built from it, the top solid level for given
   // masks of that form; nullptr for other masks (the fields are read)
   const float* mask_src;
+  // the one-launch SOR: 1 used where the grid fits and is uniform in i and j
+  // (2: always by tickets), its boxes, workspace and uniform coefficients
+  int res_on, res_uniform;
+  ResShape res;
+  unsigned long long* res_mem;
+  float res_c2, res_c3;
 };
 
+// The one-launch SOR (k_sor_res.hip): the boxes of a domain on ncu compute
+// units (false: it does not fit) and the 8-byte words of its workspace.
+bool res_shape(const Grid& g, const SplitGrid& s, int ncu, ResShape* out);
+long res_words(const Grid& g, const SplitGrid& s, const ResShape& h);
+inline bool use_res(const DevDomain& d) { return d.res_on && d.res_uniform && d.cn1_separable; }
+// One solve: from the field p and its ghosts (zero: from 0) to iterate set 1.
+void launch_sor_res(const DevDomain& d, const SplitBufs& sb, int nmaxp, float pjuge, float omega, bool zero);
 int sor_kchunk(const Grid& g, const SplitGrid& s, int target);
 int sor_parts_needed(const Grid& g, const SplitGrid& s, int target);
 int sor_fused_kchunk(const Grid& g, const SplitGrid& s, int target, int ncu);

@@ -283,6 +283,7 @@ struct les_domain {
   float* inflow_dev = nullptr;
   std::vector<float> mhost;         // metric pack on host
   int moff[NMETRICS] = {};          // offset of each metric in the pack
+  int lev_off = 0;                  // offset of Metrics::lev4
   bool mdirty = true;
   bool have_inflow = false;
   float* split = nullptr;           // colour-split SOR arrays
@@ -480,6 +481,25 @@ void derive(les_domain* D) {
     D->mhost[D->moff[MCNBY] + j + 1] = 2.0f / (metric_at(D, MDYS, j - 1) * metric_at(D, MDYS, j));
   for (int k = 1; k <= g.km; k++)
     D->mhost[D->moff[MCNCZ] + k + 1] = 2.0f / (metric_at(D, MDZS, k - 1) * metric_at(D, MDZS, k));
+  // uniform in i and j (the reference's grid is, grid.f95:36-38, 67-69): the
+  // one-launch SOR takes cn2l = cn2s and cn3l = cn3s as constants and cn1 per level
+  auto flat = [&](int mi, int n, float x) {
+    for (int q = 1; q <= n; q++)
+      if (metric_at(D, mi, q) != x) return false;
+    return true;
+  };
+  const float c2 = metric_at(D, MCN2L, 1), c3 = metric_at(D, MCN3L, 1);
+  const float ax = metric_at(D, MCNAX, 1), by = metric_at(D, MCNBY, 1);
+  D->d.res_uniform = flat(MCN2L, g.im, c2) && flat(MCN2S, g.im, c2) && flat(MCN3L, g.jm, c3) &&
+                     flat(MCN3S, g.jm, c3) && flat(MCNAX, g.im, ax) && flat(MCNBY, g.jm, by);
+  D->d.res_c2 = c2;
+  D->d.res_c3 = c3;
+  for (int k = 1; k <= g.km; k++) {
+    float* l = D->mhost.data() + D->lev_off + 4 * k;
+    l[0] = metric_at(D, MCN4L, k);
+    l[1] = metric_at(D, MCN4S, k);
+    l[2] = 1.0f / ((ax + by) + metric_at(D, MCNCZ, k));
+  }
   double area = 0.0;
   for (int k = 1; k <= g.km; k++) {
     const float dz = metric_at(D, MDZN, k);
@@ -541,6 +561,46 @@ int nmaxp_default = 50;
 float pjuge_default = 1.0e-4f;
 float omega_default = 1.0f;
 
+// The solves of k_sor_res need every compute unit they were cut for at once:
+// two of them running side by side would each hold units the other waits
+// for, until both fall back to their slow form.  So in this process the
+// enqueued work holding one is ordered, per device, after the work holding
+// the one before, when that is on another stream: an event recorded there
+// now.  The lock is held while the work is enqueued.
+std::mutex g_res_mu;
+struct ResLast {
+  hipStream_t stream = nullptr;
+  hipEvent_t ev = nullptr;
+};
+std::map<int, ResLast> g_res_last;
+
+struct ResOrder {
+  std::unique_lock<std::mutex> lk;
+  hipError_t err = hipSuccess;
+  ResOrder(bool on, hipStream_t s) {
+    if (!on) return;
+    lk = std::unique_lock<std::mutex>(g_res_mu);
+    int dev = 0;
+    if ((err = hipGetDevice(&dev)) != hipSuccess) return;
+    ResLast& l = g_res_last[dev];
+    if (l.stream && l.stream != s) {
+      std::lock_guard<std::recursive_mutex> ck(g_capture_mu);  // neither stream is being captured
+      if (!l.ev) err = hipEventCreateWithFlags(&l.ev, hipEventDisableTiming);
+      if (err == hipSuccess) err = hipEventRecord(l.ev, l.stream);
+      if (err == hipSuccess) err = hipStreamWaitEvent(s, l.ev, 0);
+      if (err != hipSuccess) return;
+    }
+    l.stream = s;
+  }
+};
+
+// The stream goes away (its work is complete).
+void res_forget(hipStream_t s) {
+  std::lock_guard<std::mutex> lk(g_res_mu);
+  for (auto& kv : g_res_last)
+    if (kv.second.stream == s) kv.second.stream = nullptr;
+}
+
 void timer_free(les_domain* D) {
   Timer* T = (Timer*)D->d.timer;
   if (!T) return;
@@ -564,6 +624,8 @@ void domain_free(les_domain* D) {
   dev_release(D->d.ctrl);
   dev_release(D->d.partials);
   dev_release(D->d.dc64);
+  dev_release(D->d.res_mem);
+  res_forget(D->d.stream);
   stream_destroy(D->d.stream);
   delete D;
 }
@@ -634,6 +696,9 @@ int domain_alloc(int im, int jm, int km, les_domain** out) {
     D->moff[mi] = off;
     off += axis_n(D, kMetrics[mi].axis) + 4;
   }
+  off = (off + 15) / 16 * 16;  // scalar loads of whole levels
+  D->lev_off = off;
+  off += 4 * (km + 1 + 24);  // levels 0..km and a box's padding
   D->mhost.assign(off, 0.0f);
   e = dev_alloc(&D->mbuf, off * sizeof(float));
   if (e != hipSuccess) return bail(std::string("metric allocation: ") + hipGetErrorString(e));
@@ -654,6 +719,7 @@ int domain_alloc(int im, int jm, int km, les_domain** out) {
   m.cnax = D->mbuf + D->moff[MCNAX];
   m.cnby = D->mbuf + D->moff[MCNBY];
   m.cncz = D->mbuf + D->moff[MCNCZ];
+  m.lev4 = D->mbuf + D->lev_off;
   m.inflow = nullptr;
   // reduction scratch: reduction partials, then the four SOR partial slots
   // at least the 2 x 256 slots of the bondv1 outflow's block max/min
@@ -687,6 +753,18 @@ int domain_alloc(int im, int jm, int km, les_domain** out) {
     if (hipGetDevice(&dev) == hipSuccess &&
         hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess)
       D->d.ncu = ncu;
+  }
+  // the one-launch SOR, unless a launch shape of the others is asked for
+  D->d.res_on = env_int("LES_SOR_RESIDENT", 1);
+  for (const char* v : {"LES_SOR_ROWS", "LES_SOR_FUSED", "LES_SOR_KCHUNK"})
+    if (getenv(v)) D->d.res_on = 0;
+  if (D->d.res_on && !res_shape(D->d.g, D->d.sg, D->d.ncu > 0 ? D->d.ncu : 256, &D->d.res)) D->d.res_on = 0;
+  if (D->d.res_on) {
+    const size_t nb = (size_t)res_words(D->d.g, D->d.sg, D->d.res) * 8;
+    e = dev_alloc(&D->d.res_mem, nb);
+    if (e == hipSuccess) e = hipMemsetAsync(D->d.res_mem, 0, nb, D->d.stream);
+    if (e != hipSuccess) return bail(std::string("SOR workspace allocation: ") + hipGetErrorString(e));
+    D->bytes += (long long)nb;
   }
   // SOR partial slots for any k chunk of the fused iteration (down to one
   // level per block) and for the colour sweeps
@@ -779,6 +857,9 @@ int run_step(les_domain* D, int n, int nmax) {
   }
   return 0;
 }
+
+// Whether the domain's press launches the one-launch SOR.
+bool press_res(const les_domain* D) { return D->d.press_mode == 0 && D->d.nmaxp >= 1 && use_res(D->d); }
 
 // Stages velnw..adam of a step (as run_step), then press: whole when the
 // domain's SOR cannot be batched, else its first part (the right-hand side
@@ -1340,6 +1421,9 @@ int les_press(int km, int jm, int im, float* rhs, const float* u, const float* d
   D->d.nmaxp = nmaxp_default;
   D->d.pjuge = pjuge_default;
   D->d.omega = omega_default;
+  if (flush_metrics(D)) return 1;
+  ResOrder order(press_res(D), D->d.stream);
+  HIP_TRY(order.err);
   return run_stage(D, 6, n, nmax);
 }
 
@@ -1654,6 +1738,16 @@ long long les_domain_bytes_needed(int im, int jm, int km) {
   long long b = 0;
   for (int f = 0; f < kLazyFirst; f++) b += (kFields[f].kind == K2D ? sk : n3) * 4;
   b += (10 * cs + 2 * cp * jm) * 4;  // colour-split SOR arrays and their two scratch planes
+  {
+    int dev = 0, ncu = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || ncu <= 0)
+      ncu = 256;
+    Grid g{im, jm, km, (int)sj, 0};
+    SplitGrid s{(int)nt, (int)cp, 0};
+    ResShape h;
+    if (res_shape(g, s, ncu, &h)) b += 8LL * res_words(g, s, h);  // the one-launch SOR
+  }
   b += ((long long)im * jm + km) * 4;  // the masks' column values and level thresholds
   return b + (1LL << 20);  // metrics, partial sums, control block (bounded by 1 MiB here)
 }
@@ -1668,6 +1762,9 @@ int les_domain_destroy(les_domain* D) {
 
 int les_domain_stage(les_domain* D, int stage, int n, int nmax) {
   if (!live_has(D)) return fail("null, unknown or destroyed domain");
+  if (flush_metrics(D)) return 1;
+  ResOrder order(stage == 6 && press_res(D), D->d.stream);
+  HIP_TRY(order.err);
   return run_stage(D, stage, n, nmax);
 }
 
@@ -1714,6 +1811,9 @@ static int step_graph(les_domain* D, int n, int nmax) {
 
 int les_domain_step(les_domain* D, int n, int nmax) {
   if (!live_has(D)) return fail("null, unknown or destroyed domain");
+  if (flush_metrics(D)) return 1;  // may allow or rule out the one-launch SOR
+  ResOrder order(press_res(D), D->d.stream);
+  HIP_TRY(order.err);
   if (D->use_graph && n != 1 && !D->d.timer) return step_graph(D, n, nmax);
   return run_step(D, n, nmax);
 }
@@ -1924,6 +2024,7 @@ void batch_free(les_batch* B) {
   for (hipEvent_t e : B->tail_done) hipEventDestroy(e);
   if (B->fork) hipEventDestroy(B->fork);
   if (B->sor_done) hipEventDestroy(B->sor_done);
+  res_forget(B->stream);
   stream_destroy(B->stream);
   delete B;
 }
@@ -2071,6 +2172,7 @@ int batch_enqueue(les_batch* B, const int* ns, const int* nmaxs, bool capturing)
     if (B->full[q] && ns[q] == 1) staged = false;
   HIP_TRY(hipEventRecord(B->fork, B->stream));
   std::vector<char> split(nd, 0);
+  int res_prev = -1;
   for (size_t q = 0; q < nd; q++) {
     les_domain* D = B->doms[q];
     D->rhs_lazy = D->d.press_mode == 0;  // a batched press also leaves the split rhs equal to rhs
@@ -2083,6 +2185,10 @@ int batch_enqueue(les_batch* B, const int* ns, const int* nmaxs, bool capturing)
       continue;
     }
     HIP_TRY(hipStreamWaitEvent(D->d.stream, B->fork, 0));
+    if (!B->full[q] && press_res(D)) {  // those running the one-launch SOR step one after the other
+      if (res_prev >= 0) HIP_TRY(hipStreamWaitEvent(D->d.stream, B->head_done[res_prev], 0));
+      res_prev = (int)q;
+    }
     if (B->full[q]) {
       bool sp = false;
       if (run_step_head(D, ns[q], nmaxs[q], B->sor_kc, B->sor_ty, B->sor_tw, &sp)) return 1;
@@ -2185,6 +2291,10 @@ int les_batch_step(les_batch* B, const int* ns, const int* nmaxs) {
     if (flush_metrics(D)) return 1;  // synchronous: not under capture
     D->rhs_lazy = D->d.press_mode == 0;
   }
+  bool res = false;  // a domain stepping whole on its own stream runs the one-launch SOR
+  for (size_t q = 0; q < B->doms.size(); q++) res = res || (!B->full[q] && press_res(B->doms[q]));
+  ResOrder order(res, B->stream);
+  HIP_TRY(order.err);
   bool replay = B->use_graph != 0;
   for (size_t q = 0; q < B->doms.size(); q++) replay = replay && ns[q] != 1;
   if (!replay) return batch_enqueue(B, ns, nmaxs, false);
