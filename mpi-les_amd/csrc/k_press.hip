@@ -1954,15 +1954,18 @@ __global__ __launch_bounds__(256) void k_dc_norm(const double* __restrict__ part
   if (threadIdx.x == 0) {
     hist[step] = s;
     ctrl->dc_norms = step + 1;
+    res_begin(ctrl);  // the inner iterations may run in one launch
     if (s < (double)pjuge || !(s == s) || s > 1.0e300) ctrl->dc_done = 1;
   }
 }
 
-// P64 += e (the inner solve's last iterate, in iterate set `set`), unless
-// the defect met the stop threshold
+// P64 += e (the inner solve's last iterate, in iterate set `set`, or where
+// the inner solve left it when set < 0), unless the defect met the stop
+// threshold
 __global__ __launch_bounds__(NT) void k_dc_correct(Grid g, SplitGrid s, SplitBufs sb, double* __restrict__ P64,
                                                    int set, const Ctrl* ctrl) {
   if (ctrl->dc_done) return;  // uniform
+  if (set < 0) set = ctrl->p_final;
   const int i = 1 + blockIdx.x * BX + threadIdx.x, j = 1 + blockIdx.y * BY + threadIdx.y;
   if (i > g.im || j > g.jm) return;
   const int t = (i - 1) >> 1;
@@ -2205,11 +2208,13 @@ static void launch_sor_iter(const DevDomain& d, const SplitBufs& sb, int l, floa
 static void launch_press_dc(const DevDomain& d, const SplitBufs& sb, int gx, int gy, int gz, int nred) {
   const Grid& g = d.g;
   const SplitGrid& s = d.sg;
-  // the inner iterations two per launch where the domain's SOR runs so
-  // (iterate sets rotating over three from set 0, which k_dc_defect clears),
-  // else one per launch; they never stop on their own (threshold 0)
+  // the inner iterations in one launch or two per launch where the domain's
+  // SOR runs so (iterate sets rotating over three from set 0, which
+  // k_dc_defect clears), else one per launch; they never stop on their own
+  // (threshold 0).  16 steps at 256x256x64 with the iterations two per launch
+  // take 47.1 ms, in one launch per inner solve 36.6.
   const SorShape hp = sor_shape(d);
-  const bool pairs = hp.rows == 4;
+  const bool res = press_resident(d), pairs = hp.rows == 4;
   const SorShape h = pairs ? hp : sor_shape_single(d);
   double* P64 = d.dc64;
   double* R64 = d.dc64 + d.n3;
@@ -2228,7 +2233,10 @@ static void launch_press_dc(const DevDomain& d, const SplitBufs& sb, int gx, int
     TIMED(d, KC_RHS, hipLaunchKernelGGL(k_dc_norm, dim3(1), dim3(256), 0, d.stream, (const double*)d.partials, nred,
                                         hist, o, d.ctrl, d.pjuge));
     int set = d.dc_inner & 1;  // the iterate set holding the inner result
-    if (pairs)
+    if (res) {
+      launch_sor_res(di, sb, d.dc_inner, 0.0f, di.omega, true);
+      set = -1;
+    } else if (pairs)
       set = launch_sor_pairs(di, sb, h, 0.0f, 1, d.dc_inner, 0, nullptr).out_set;
     else
       for (int l = 1; l <= d.dc_inner; l++) launch_sor_iter(di, sb, l, 0.0f, h, h.nparts);
@@ -2516,7 +2524,7 @@ void launch_press(const DevDomain& d, float dt) {
   const int nred = gx * gy * gz;
   SplitBufs sb = d.sb;
   if (d.cn1_separable) sb.cn1[0] = sb.cn1[1] = nullptr;
-  const bool res = d.press_mode == 0 && d.nmaxp >= 1 && use_res(d);
+  const bool res = d.press_mode == 0 && press_resident(d);
   if (res || (d.press_mode == 0 && d.sor_fused && d.nmaxp >= 1 && sor_shape(d).rows == 4)) {
     // two iterations per launch: the head in one pass (k_rhs_head), the mean
     // removal over the split rhs alone (k_rhs_sub); the launch of iterations

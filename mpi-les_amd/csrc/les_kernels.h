@@ -128,6 +128,10 @@ struct DevDomain {
 bool res_shape(const Grid& g, const SplitGrid& s, int ncu, ResShape* out);
 long res_words(const Grid& g, const SplitGrid& s, const ResShape& h);
 inline bool use_res(const DevDomain& d) { return d.res_on && d.res_uniform && d.cn1_separable; }
+// Whether a press runs it, for its solve or for the inner ones of mode 1.
+inline bool press_resident(const DevDomain& d) {
+  return use_res(d) && (d.press_mode == 0 ? d.nmaxp : d.dc_inner) >= 1;
+}
 // One solve: from the field p and its ghosts (zero: from 0) to iterate set 1.
 void launch_sor_res(const DevDomain& d, const SplitBufs& sb, int nmaxp, float pjuge, float omega, bool zero);
 int sor_kchunk(const Grid& g, const SplitGrid& s, int target);

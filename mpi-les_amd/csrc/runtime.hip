@@ -858,9 +858,6 @@ int run_step(les_domain* D, int n, int nmax) {
   return 0;
 }
 
-// Whether the domain's press launches the one-launch SOR.
-bool press_res(const les_domain* D) { return D->d.press_mode == 0 && D->d.nmaxp >= 1 && use_res(D->d); }
-
 // Stages velnw..adam of a step (as run_step), then press: whole when the
 // domain's SOR cannot be batched, else its first part (the right-hand side
 // and SOR iteration 1, with the batch's SOR k chunk kc and tile rows ty).
@@ -1422,7 +1419,7 @@ int les_press(int km, int jm, int im, float* rhs, const float* u, const float* d
   D->d.pjuge = pjuge_default;
   D->d.omega = omega_default;
   if (flush_metrics(D)) return 1;
-  ResOrder order(press_res(D), D->d.stream);
+  ResOrder order(press_resident(D->d), D->d.stream);
   HIP_TRY(order.err);
   return run_stage(D, 6, n, nmax);
 }
@@ -1763,7 +1760,7 @@ int les_domain_destroy(les_domain* D) {
 int les_domain_stage(les_domain* D, int stage, int n, int nmax) {
   if (!live_has(D)) return fail("null, unknown or destroyed domain");
   if (flush_metrics(D)) return 1;
-  ResOrder order(stage == 6 && press_res(D), D->d.stream);
+  ResOrder order(stage == 6 && press_resident(D->d), D->d.stream);
   HIP_TRY(order.err);
   return run_stage(D, stage, n, nmax);
 }
@@ -1812,7 +1809,7 @@ static int step_graph(les_domain* D, int n, int nmax) {
 int les_domain_step(les_domain* D, int n, int nmax) {
   if (!live_has(D)) return fail("null, unknown or destroyed domain");
   if (flush_metrics(D)) return 1;  // may allow or rule out the one-launch SOR
-  ResOrder order(press_res(D), D->d.stream);
+  ResOrder order(press_resident(D->d), D->d.stream);
   HIP_TRY(order.err);
   if (D->use_graph && n != 1 && !D->d.timer) return step_graph(D, n, nmax);
   return run_step(D, n, nmax);
@@ -2185,7 +2182,7 @@ int batch_enqueue(les_batch* B, const int* ns, const int* nmaxs, bool capturing)
       continue;
     }
     HIP_TRY(hipStreamWaitEvent(D->d.stream, B->fork, 0));
-    if (!B->full[q] && press_res(D)) {  // those running the one-launch SOR step one after the other
+    if (!B->full[q] && press_resident(D->d)) {  // those running the one-launch SOR step one after the other
       if (res_prev >= 0) HIP_TRY(hipStreamWaitEvent(D->d.stream, B->head_done[res_prev], 0));
       res_prev = (int)q;
     }
@@ -2292,7 +2289,7 @@ int les_batch_step(les_batch* B, const int* ns, const int* nmaxs) {
     D->rhs_lazy = D->d.press_mode == 0;
   }
   bool res = false;  // a domain stepping whole on its own stream runs the one-launch SOR
-  for (size_t q = 0; q < B->doms.size(); q++) res = res || (!B->full[q] && press_res(B->doms[q]));
+  for (size_t q = 0; q < B->doms.size(); q++) res = res || (!B->full[q] && press_resident(B->doms[q]->d));
   ResOrder order(res, B->stream);
   HIP_TRY(order.err);
   bool replay = B->use_graph != 0;

@@ -156,3 +156,35 @@ def test_domains_in_turn_and_a_grid_that_does_not_qualify():
     assert np.array_equal(a.press_stats()["sor"], b.press_stats()["sor"])  # the same kernel: the same order of sums
     a.close()
     b.close()
+
+
+@pytest.mark.parametrize("mode", [1, 2], ids=["resident", "tickets"])
+@pytest.mark.parametrize("dims,outer,inner,omega", [((40, 28, 14), 1, 1, 1.0), ((61, 27, 13), 3, 2, 1.0),
+                                                    ((96, 64, 32), 2, 50, 1.0), ((40, 28, 14), 4, 7, 1.6),
+                                                    ((40, 28, 14), 6, 20, 1.0)])
+def test_inner_solves_of_the_defect_correction(dims, outer, inner, omega, mode):
+    """The inner solves from zero (the last case meets the stop threshold of
+    step 1 at its fourth norm, so later outer steps are skipped)."""
+    base = dataclasses.replace(setup_gen.small_workload(*dims, seed=5), pjuge=1e-30)
+    if outer == 6:
+        probe = _domain(setup_gen.build(base, dense=False), LES_SOR_RESIDENT=0)
+        probe.set_press_mode(1, outer=outer, inner=inner)
+        probe.step(1, 3)
+        h = probe.press_stats()["sor"]
+        probe.close()
+        assert h[3] < min(h[:3])
+        base = dataclasses.replace(base, pjuge=float(np.sqrt(h[3] * min(h[:3]))))
+    s = setup_gen.build(base, dense=False)
+    print(f"\n[sor res dc] {dims} {outer}x{inner} omega {omega} mode {mode}", flush=True)
+    ref, res = _domain(s, LES_SOR_RESIDENT=0), _domain(s, LES_SOR_RESIDENT=mode)
+    for d in (ref, res):
+        d.set_press_mode(1, outer=outer, inner=inner)
+        d.set_press_omega(omega)
+    res.set_graph(True)
+    for n in range(1, 4):
+        ref.step(n, 3)
+        res.step(n, 3)
+        st = _same(ref, res, n)
+        assert outer != 6 or n > 1 or st["iters"] == 4, st["iters"]
+    ref.close()
+    res.close()
