@@ -319,7 +319,8 @@ long long les_domain_bytes(const les_domain* d);
  * Domains with a batchable whole step (fused reference SOR, separable cn1,
  * even jm, velfg+feedbf and les+adam fused) run every stage as one launch
  * for all of them: each block runs its own domain's stage on that domain's
- * grid, and the SOR iterations 2..nmaxp run as one launch per iteration
+ * grid, and the SOR runs as one launch (domains whose solve fits the device's
+ * registers, side by side), or iterations 2..nmaxp as one launch per iteration
  * with one k chunk for the batch (LES_BATCH_SOR_KCHUNK and
  * LES_BATCH_SOR_TILE_ROWS override it).  A step in which such a domain has
  * n == 1 runs its stages on its own stream and only the SOR iterations

@@ -146,7 +146,7 @@ __global__ __launch_bounds__(256) void k_finalize(const double* __restrict__ par
 __device__ __forceinline__ void rhs_split_body(const VBlk& vb, const Grid& g, const SplitGrid& s,
                                                float* __restrict__ rhs, const float* __restrict__ p,
                                                const float* __restrict__ cn1, const SplitBufs& sb,
-                                               Ctrl* ctrl) {
+                                               Ctrl* ctrl, bool copy_p = true) {
   const int i = 1 + vb.x * BX + threadIdx.x, j = 1 + vb.y * BY + wave_row();
   if (i > g.im || j > g.jm) return;
   const double av = ctrl->rhsav;
@@ -162,6 +162,7 @@ __device__ __forceinline__ void rhs_split_body(const VBlk& vb, const Grid& g, co
     rhs[c] = r;
     const int q = cix(s, t, j, k);
     sb.rhs[col][q] = r;
+    if (!copy_p) continue;  // k_sor_res reads p and its ghosts themselves
     const float pc = p[c];
     sb.p[0][col][q] = pc;
     if (sb.cn1[0]) sb.cn1[col][q] = cn1[c];
@@ -2443,11 +2444,12 @@ __global__ __launch_bounds__(NT) void kb_rhs(const BatchDom* __restrict__ bd, co
 __global__ __launch_bounds__(256) void kb_finalize(const BatchDom* __restrict__ bd, int what) {
   const BatchDom& B = bd[blockIdx.x];
   finalize_body(B.d.partials, B.nred, B.d.ctrl, what, B.d.area);
+  if (what == 0 && threadIdx.x == 0) res_begin(B.d.ctrl);
 }
 __global__ __launch_bounds__(NT) void kb_rhs_split(const BatchDom* __restrict__ bd,
                                                    const StageSpan* __restrict__ sp, int nd) {
   BATCH_BLOCK(BS_SPLIT, false);
-  rhs_split_body(vb, d.g, d.sg, d.F.rhs, d.F.p, d.F.cn1, B.sb, d.ctrl);
+  rhs_split_body(vb, d.g, d.sg, d.F.rhs, d.F.p, d.F.cn1, B.sb, d.ctrl, B.nparts_last > 0);
 }
 __global__ __launch_bounds__(FNT) __attribute__((amdgpu_waves_per_eu(8, 8))) void kb_sor_entry(
     const BatchDom* __restrict__ bd, const StageSpan* __restrict__ sp, int nd) {
@@ -2458,7 +2460,7 @@ __global__ __launch_bounds__(FNT) __attribute__((amdgpu_waves_per_eu(8, 8))) voi
 // one block per domain
 __global__ __launch_bounds__(256) void kb_sor_final(const BatchDom* __restrict__ bd) {
   const BatchDom& B = bd[blockIdx.x];
-  sor_final_body(B.sb, B.d.ctrl, B.d.nmaxp, B.nparts_last);
+  if (B.nparts_last > 0) sor_final_body(B.sb, B.d.ctrl, B.d.nmaxp, B.nparts_last);
 }
 __global__ __launch_bounds__(NT) void kb_pav(const BatchDom* __restrict__ bd, const StageSpan* __restrict__ sp,
                                              int nd) {
@@ -2472,7 +2474,7 @@ __global__ __launch_bounds__(NT) void kb_padj(const BatchDom* __restrict__ bd, c
 }
 #undef BATCH_BLOCK
 
-void press_batch_spans(const DevDomain& d, int kc, int ty, int tw, int nzb, BatchDom* e, StageSpan* sp) {
+void press_batch_spans(const DevDomain& d, bool res, int kc, int ty, int tw, int nzb, BatchDom* e, StageSpan* sp) {
   const Grid& g = d.g;
   const int gx = (g.im + BX - 1) / BX, gy = (g.jm + BY - 1) / BY;
   const int gz = kblocks(gx, gy, g.km, kMaxRedBlocks);
@@ -2485,13 +2487,13 @@ void press_batch_spans(const DevDomain& d, int kc, int ty, int tw, int nzb, Batc
   e->ntj1 = h1.ntj;
   e->kc1 = h1.kc;
   e->nparts1 = h1.nparts;
-  e->nparts_last = d.nmaxp == 1 ? h1.nparts : h.nparts;
+  e->nparts_last = res ? 0 : d.nmaxp == 1 ? h1.nparts : h.nparts;
   const int px = (g.im + 2 + BX - 1) / BX, py = (g.jm + 2 + BY - 1) / BY;
   // the reductions keep their own grids (their partial sums are the domain's
   // own); the copies may run longer k runs per block
   sp[BS_RHS] = {0, gx, gy, gz};
   sp[BS_SPLIT] = {0, gx, gy, nzb > 0 ? std::min(nzb, g.km) : g.km};
-  sp[BS_SOR1] = {0, h1.nparts, 1, 1};
+  sp[BS_SOR1] = {0, res ? 0 : h1.nparts, 1, 1};
   sp[BS_PAV] = {0, gx, gy, gz};
   sp[BS_PADJ] = {0, px, py, nzb > 0 ? std::min(nzb, g.km + 2) : g.km + 2};
 }
@@ -2505,10 +2507,11 @@ void launch_press_batch(const StageBatch& b, int part, hipStream_t stream, bool 
     hipLaunchKernelGGL(kb_rhs, nb(BS_RHS), blk(), 0, stream, bd, sp, nd);
     hipLaunchKernelGGL(kb_finalize, dim3((unsigned)nd), dim3(256), 0, stream, bd, 0);
     hipLaunchKernelGGL(kb_rhs_split, nb(BS_SPLIT), blk(), 0, stream, bd, sp, nd);
+    if (b.nblocks[BS_SOR1] == 0) return;  // every domain solves in one launch
     hipLaunchKernelGGL(kb_sor_entry, nb(BS_SOR1), dim3(FX, FY), 3 * (size_t)(b.kc1max + 2) * sizeof(float), stream,
                        bd, sp, nd);
   } else {
-    if (!pairs)  // with pairs: launch_sor_pair_batch ran the closing stop test
+    if (!pairs && b.nblocks[BS_SOR1] > 0)  // with pairs: launch_sor_pair_batch ran the closing stop test
       hipLaunchKernelGGL(kb_sor_final, dim3((unsigned)nd), dim3(256), 0, stream, bd);
     hipLaunchKernelGGL(kb_pav, nb(BS_PAV), blk(), 0, stream, bd, sp, nd);
     hipLaunchKernelGGL(kb_finalize, dim3((unsigned)nd), dim3(256), 0, stream, bd, 1);

@@ -756,10 +756,26 @@ __device__ __forceinline__ void res_block(ConstArgs a0, const int bid) {
   }
 }
 
+// One solve, of the arguments a, or (nd > 0) those of a batch: domain e's
+// arguments are tab[e] and its blocks start at b0[e].  The domains of a batch
+// share the device side by side, each with boxes of its own and a handshake of
+// its own: 9 domains of 96..160 x 96..160 x 64 solve 50
+// iterations in 1165 us, one iteration of all of them per launch took 2090.
 template <int CLS, int BK, bool OM1, bool ODD>
-__global__ __launch_bounds__(kResNT, 2 * kResClass[CLS].per) void k_sor_res(ResArgs a) {
+__global__ __launch_bounds__(kResNT, 2 * kResClass[CLS].per) void k_sor_res(ResArgs a,
+                                                                             const ResArgs* __restrict__ tab,
+                                                                             const int* __restrict__ b0, int nd) {
   (void)a;  // the kernel argument segment starts with it
-  res_block<CLS, BK, OM1, ODD>((ConstArgs)__builtin_amdgcn_kernarg_segment_ptr(), (int)blockIdx.x);
+  ConstArgs at = (ConstArgs)__builtin_amdgcn_kernarg_segment_ptr();
+  int bid = (int)blockIdx.x;
+  if (nd > 0) {
+    int e = 0;
+    for (int r = 1; r < nd; r++)
+      if ((int)blockIdx.x >= b0[r]) e = r;
+    at = (ConstArgs)(unsigned long long)(tab + e);
+    bid -= b0[e];
+  }
+  res_block<CLS, BK, OM1, ODD>(at, bid);
 }
 
 }  // namespace
@@ -767,48 +783,151 @@ __global__ __launch_bounds__(kResNT, 2 * kResClass[CLS].per) void k_sor_res(ResA
 // Microseconds of one sweep of a cut, as a model: the sweep of a unit's boxes
 // (80 cycles per level and wave of a SIMD, no less than the latency of a wave
 // alone), the exchange (latency, and words per unit), and what a box of two
-// hides of it.
-static double res_cost(int waves, int kl, int nb, int words, int cls, int units) {
-  const int on = nb > units ? 2 : 1;  // boxes on the fullest unit
+// hides of it.  on: boxes on the fullest unit.
+static double res_cost(int waves, int kl, int nb, int words, int on) {
   const double sweep = std::max(0.034 * ((on * waves + 3) / 4), 0.055) * kl + 0.3 + 0.05 * waves * on;
   const double cross = nb > 1 ? 1.5 + 0.35 * on * words / 1024 : 0.0;
-  (void)cls;
   return on == 1 ? sweep + cross : std::max(sweep, 0.6 * sweep + cross);
+}
+
+static int up(int a, int b) { return (a + b - 1) / b; }
+static int res_face_words(const ResShape& h) { return 2 * (h.ntx > 1 ? h.tj * h.kl : 0) + 2 * h.tp * h.kl; }
+// The threads a launch has: whole waves.
+static void res_threads(ResShape* h, int nthr) {
+  h->nthr = nthr;
+  h->nq = up(res_face_words(*h), nthr);
+  h->iw = h->nq * nthr + 2 * kResNT;
+}
+
+// Calls f(shape, halo words) for every cut of a domain into at most nmax boxes
+// of class cls with klo < levels <= khi.
+template <class F>
+static void res_cuts(const Grid& g, const SplitGrid& s, int cls, int nmax, int klo, int khi, F f) {
+  const ResClass C = kResClass[cls];
+  for (int ntz = std::max(1, up(g.km, khi)); ntz <= std::min(g.km, nmax); ntz++) {
+    const int kl = up(g.km, ntz);
+    if (kl <= klo) break;
+    if (kl > khi || (ntz > 1 && kl == up(g.km, ntz - 1))) continue;
+    for (int ntx = 1; ntx <= s.nt && ntx * ntz <= nmax; ntx++) {
+      const int tp = up(s.nt, ntx);
+      if (tp > kResNT || (ntx > 1 && tp == up(s.nt, ntx - 1))) continue;
+      for (int nty = std::max(1, up(g.jm, kResNT / tp)); nty <= g.jm && ntx * nty * ntz <= nmax; nty++) {
+        const int tj = up(g.jm, nty);
+        if (tp * tj > kResNT || (nty > 1 && tj == up(g.jm, nty - 1))) continue;
+        if ((tp + 2) * (tj + 2 + ((g.jm & 1) ? 4 : 0)) >= C.plane) continue;
+        ResShape h{ntx, nty, ntz, tp, tj, kl, ntx * nty * ntz, 0, 0, cls, 0};
+        // enough waves for the columns and for the halo words
+        const int wds = res_face_words(h);
+        const int nthr = up(std::max(tp * tj, up(wds, C.words)), kWave) * kWave;
+        if (nthr > kResNT) continue;
+        res_threads(&h, nthr);
+        f(h, wds + (ntz > 1 ? 2 * nthr : 0));
+      }
+    }
+  }
 }
 
 // The cut of a domain into boxes with the least modelled time.  False when
 // no cut fits (about 12 million cells on 256 units).
 bool res_shape(const Grid& g, const SplitGrid& s, int units, ResShape* out) {
   double best = -1.0;
-  const auto up = [](int a, int b) { return (a + b - 1) / b; };
+  for (int cls = 0; cls < 2; cls++)  // one block runs the monitor
+    res_cuts(g, s, cls, kResClass[cls].per * units - 1, 0, kResClass[cls].levels, [&](const ResShape& h, int wds) {
+      const double c = res_cost(h.nthr / kWave, h.kl, h.nb, wds, h.nb > units ? 2 : 1);
+      if (best < 0.0 || c < best) {
+        best = c;
+        *out = h;
+      }
+    });
+  return best >= 0.0;
+}
+
+// One launch for the domains ds (indices into all): the kernel (class and
+// levels) and one cut of each, such that all boxes run at once, with the least
+// modelled time of the slowest domain.  From its fewest boxes each domain takes
+// more while it is the slowest and they fit.  Returns the time, negative when
+// no kernel holds them all.
+static double res_batch_cut(const DevDomain* const* all, const std::vector<int>& ds, int units, ResShape* shapes) {
+  struct Cut {
+    ResShape h;
+    double cost;
+  };
+  double best = -1.0;
   for (int cls = 0; cls < 2; cls++) {
-    const ResClass C = kResClass[cls];
-    const int nmax = C.per * units - 1;  // one block runs the monitor
-    for (int ntz = 1; ntz <= std::min(g.km, nmax); ntz++) {
-      const int kl = up(g.km, ntz);
-      if (kl > C.levels || (ntz > 1 && kl == up(g.km, ntz - 1))) continue;
-      for (int ntx = 1; ntx <= s.nt && ntx * ntz <= nmax; ntx++) {
-        const int tp = up(s.nt, ntx);
-        if (tp > kResNT || (ntx > 1 && tp == up(s.nt, ntx - 1))) continue;
-        for (int nty = std::max(1, up(g.jm, kResNT / tp)); nty <= g.jm && ntx * nty * ntz <= nmax; nty++) {
-          const int tj = up(g.jm, nty);
-          if (tp * tj > kResNT || (nty > 1 && tj == up(g.jm, nty - 1))) continue;
-          if ((tp + 2) * (tj + 2 + ((g.jm & 1) ? 4 : 0)) >= C.plane) continue;
-          const int ni = ntx > 1 ? tj * kl : 0, nj = tp * kl, nb = ntx * nty * ntz, wds = 2 * ni + 2 * nj;
-          // whole waves, enough for the columns and for the halo words
-          const int nthr = up(std::max(tp * tj, up(wds, C.words)), kWave) * kWave;
-          if (nthr > kResNT) continue;
-          const int nq = up(wds, nthr);
-          const double cost = res_cost(nthr / kWave, kl, nb, wds + (ntz > 1 ? 2 * nthr : 0), cls, units);
-          if (best < 0.0 || cost < best) {
-            best = cost;
-            *out = ResShape{ntx, nty, ntz, tp, tj, kl, nb, nq * nthr + 2 * kResNT, nq, cls, nthr};
-          }
+    const int cap = kResClass[cls].per * units;
+    for (int bk = 4; bk <= kResClass[cls].levels; bk += 4) {
+      std::vector<std::vector<Cut>> cuts(ds.size());  // of rising boxes and falling time
+      long total = 0;
+      bool ok = true;
+      for (size_t q = 0; q < ds.size() && ok; q++) {
+        const DevDomain& d = *all[ds[q]];
+        std::vector<Cut> v;
+        res_cuts(d.g, d.sg, cls, cap - 1, bk - 4, bk, [&](const ResShape& h, int wds) {
+          v.push_back({h, res_cost(h.nthr / kWave, h.kl, h.nb, wds, cls == 1 ? 2 : 1)});
+        });
+        std::stable_sort(v.begin(), v.end(), [](const Cut& a, const Cut& b) { return a.h.nb < b.h.nb; });
+        for (const Cut& c : v) {
+          auto& w = cuts[q];
+          if (!w.empty() && c.cost >= w.back().cost) continue;
+          if (!w.empty() && c.h.nb == w.back().h.nb)
+            w.back() = c;
+          else
+            w.push_back(c);
         }
+        ok = !cuts[q].empty();
+        if (ok) total += cuts[q][0].h.nb + 1;
+      }
+      if (!ok || total > cap) continue;
+      std::vector<size_t> at(ds.size(), 0);
+      double slow;
+      for (;;) {
+        size_t m = 0;
+        for (size_t q = 1; q < ds.size(); q++)
+          if (cuts[q][at[q]].cost > cuts[m][at[m]].cost) m = q;
+        slow = cuts[m][at[m]].cost;
+        if (at[m] + 1 == cuts[m].size()) break;
+        const long more = cuts[m][at[m] + 1].h.nb - cuts[m][at[m]].h.nb;
+        if (total + more > cap) break;
+        total += more;
+        at[m]++;
+      }
+      if (best >= 0.0 && slow >= best) continue;
+      best = slow;
+      int nthr = 0;
+      for (size_t q = 0; q < ds.size(); q++) nthr = std::max(nthr, cuts[q][at[q]].h.nthr);
+      for (size_t q = 0; q < ds.size(); q++) {
+        shapes[ds[q]] = cuts[q][at[q]].h;
+        res_threads(&shapes[ds[q]], nthr);
       }
     }
   }
-  return best >= 0.0;
+  return best;
+}
+
+double res_batch_plan(const DevDomain* const* ds, int n, int units, ResShape* shapes, std::vector<int>* group) {
+  std::vector<int> by(n);  // largest first
+  for (int q = 0; q < n; q++) by[q] = q;
+  const auto cells = [&](int q) { return (long)ds[q]->g.im * ds[q]->g.jm * ds[q]->g.km; };
+  std::stable_sort(by.begin(), by.end(), [&](int a, int b) { return cells(a) > cells(b); });
+  for (int ng = 1; ng <= n; ng++) {
+    std::vector<std::vector<int>> in(ng);  // dealt out there and back
+    for (int r = 0; r < n; r++) in[(r / ng) & 1 ? ng - 1 - r % ng : r % ng].push_back(by[r]);
+    double sum = 0.0;
+    for (const auto& v : in) {
+      const double c = res_batch_cut(ds, v, units, shapes);
+      if (c < 0.0) {
+        sum = -1.0;
+        break;
+      }
+      sum += c;
+    }
+    if (sum < 0.0) continue;
+    group->assign(n, 0);
+    for (int q = 0; q < ng; q++)
+      for (int r : in[q]) (*group)[r] = q;
+    return sum;
+  }
+  return -1.0;
 }
 
 // 8-byte words of the workspace: inboxes of both colours, the partial sums
@@ -821,31 +940,8 @@ long res_words(const Grid& g, const SplitGrid& s, const ResShape& h) {
   return 2L * h.nb * h.iw + 8L * h.nb * (h.nthr / kWave) + 8 + 4 * res_tickets(g, s);
 }
 
-template <int CLS, bool OM1, bool ODD>
-static void launch_res(const DevDomain& d, const ResArgs& a) {
-  const dim3 grid(d.res.nb + 1), blk(d.res.nthr);
-#define RES(BK)                                                                                          \
-  if (d.res.kl <= BK) {                                                                                  \
-    TIMED(d, KC_SOR, hipLaunchKernelGGL((k_sor_res<CLS, BK, OM1, ODD>), grid, blk, 0, d.stream, a));      \
-    return;                                                                                              \
-  }
-  RES(4)
-  RES(8)
-  RES(12)
-  RES(16)
-  RES(20)
-  RES(24)
-  if constexpr (CLS == 0) {
-    RES(28)
-    RES(32)
-    RES(36)
-    RES(40)
-  }
-#undef RES
-}
-
-void launch_sor_res(const DevDomain& d, const SplitBufs& sb, int nmaxp, float pjuge, float omega, bool zero) {
-  const ResShape& h = d.res;
+ResArgs res_args(const DevDomain& d, const ResShape& h, unsigned long long* mem, const SplitBufs& sb, int nmaxp,
+                 float pjuge, float omega, bool zero) {
   ResArgs a{};
   a.g = d.g;
   a.s = d.sg;
@@ -853,8 +949,8 @@ void launch_sor_res(const DevDomain& d, const SplitBufs& sb, int nmaxp, float pj
   a.sb = sb;
   a.ctrl = d.ctrl;
   a.pent = d.F.p;
-  a.slots = d.res_mem;
-  a.parts = d.res_mem + 2L * h.nb * h.iw;
+  a.slots = mem;
+  a.parts = mem + 2L * h.nb * h.iw;
   a.tparts = (double*)(a.parts + 8L * h.nb * (h.nthr / kWave) + 8);
   a.c2 = d.res_c2;
   a.c3 = d.res_c3;
@@ -872,22 +968,68 @@ void launch_sor_res(const DevDomain& d, const SplitBufs& sb, int nmaxp, float pj
   a.nb = h.nb;
   a.iw = h.iw;
   a.nq = h.nq;
-  const bool odd = (d.g.im & 1) != 0;
-  if (h.cls == 0) {
-    if (omega != 1.0f)
-      launch_res<0, false, true>(d, a);
-    else if (odd)
-      launch_res<0, true, true>(d, a);
-    else
-      launch_res<0, true, false>(d, a);
-  } else {
-    if (omega != 1.0f)
-      launch_res<1, false, true>(d, a);
-    else if (odd)
-      launch_res<1, true, true>(d, a);
-    else
-      launch_res<1, true, false>(d, a);
+  return a;
+}
+
+struct ResGrid {
+  int blocks, nthr, kl;
+  hipStream_t stream;
+  const ResArgs* tab;
+  const int* b0;
+  int nd;
+};
+
+template <int CLS, bool OM1, bool ODD>
+static void launch_res(const ResGrid& r, const ResArgs& a) {
+#define RES(BK)                                                                                                   \
+  if (r.kl <= BK) {                                                                                               \
+    hipLaunchKernelGGL((k_sor_res<CLS, BK, OM1, ODD>), dim3(r.blocks), dim3(r.nthr), 0, r.stream, a, r.tab, r.b0, \
+                       r.nd);                                                                                     \
+    return;                                                                                                       \
   }
+  RES(4)
+  RES(8)
+  RES(12)
+  RES(16)
+  RES(20)
+  RES(24)
+  if constexpr (CLS == 0) {
+    RES(28)
+    RES(32)
+    RES(36)
+    RES(40)
+  }
+#undef RES
+}
+
+static void launch_res(const ResGrid& r, const ResArgs& a, int cls, bool om1, bool odd) {
+  if (cls == 0) {
+    if (!om1)
+      launch_res<0, false, true>(r, a);
+    else if (odd)
+      launch_res<0, true, true>(r, a);
+    else
+      launch_res<0, true, false>(r, a);
+  } else {
+    if (!om1)
+      launch_res<1, false, true>(r, a);
+    else if (odd)
+      launch_res<1, true, true>(r, a);
+    else
+      launch_res<1, true, false>(r, a);
+  }
+}
+
+void launch_sor_res(const DevDomain& d, const SplitBufs& sb, int nmaxp, float pjuge, float omega, bool zero) {
+  const ResShape& h = d.res;
+  const ResArgs a = res_args(d, h, d.res_mem, sb, nmaxp, pjuge, omega, zero);
+  const ResGrid r{h.nb + 1, h.nthr, h.kl, d.stream, nullptr, nullptr, 0};
+  TIMED(d, KC_SOR, launch_res(r, a, h.cls, omega == 1.0f, (d.g.im & 1) != 0));
+}
+
+void launch_sor_res_batch(const ResBatch& b, hipStream_t stream) {
+  const ResGrid r{b.blocks, b.nthr, b.kl, stream, b.tab, b.b0, b.nd};
+  launch_res(r, ResArgs{}, b.cls, b.om1, b.odd);
 }
 
 }  // namespace les

@@ -134,6 +134,19 @@ inline bool press_resident(const DevDomain& d) {
 }
 // One solve: from the field p and its ghosts (zero: from 0) to iterate set 1.
 void launch_sor_res(const DevDomain& d, const SplitBufs& sb, int nmaxp, float pjuge, float omega, bool zero);
+// The same for a batch of domains, in one launch per group: group[q] and
+// shapes[q] of domain q.  Returns the modelled microseconds per colour sweep
+// of all of them, negative when one fits no cut.
+double res_batch_plan(const DevDomain* const* ds, int n, int units, ResShape* shapes, std::vector<int>* group);
+ResArgs res_args(const DevDomain& d, const ResShape& h, unsigned long long* mem, const SplitBufs& sb, int nmaxp,
+                 float pjuge, float omega, bool zero);
+struct ResBatch {
+  const ResArgs* tab;  // device, nd entries
+  const int* b0;       // device, first block of each
+  int nd, blocks, cls, kl, nthr;
+  bool om1, odd;       // every omega is 1; some im is odd
+};
+void launch_sor_res_batch(const ResBatch& b, hipStream_t stream);
 int sor_kchunk(const Grid& g, const SplitGrid& s, int target);
 int sor_parts_needed(const Grid& g, const SplitGrid& s, int target);
 int sor_fused_kchunk(const Grid& g, const SplitGrid& s, int target, int ncu);
@@ -208,7 +221,7 @@ struct BatchDom {
   int velfg_kc;    // k levels per thread of k_velfg_feedbf
   int ilast;       // last column bondv1 sets from the inflow (1 for n > 1)
   int ntt1, ntj1, kc1, nparts1;  // shape of SOR iteration 1 (k_sor_iter<true, true>)
-  int nparts_last;               // partial-sum slots of the launch of iteration nmaxp
+  int nparts_last;               // partial-sum slots of the launch of iteration nmaxp (0: solved in one launch)
 };
 struct StageBatch {
   const BatchDom* doms;    // device, nd entries
@@ -247,7 +260,7 @@ __device__ __forceinline__ bool batch_block(const StageSpan* __restrict__ sp, in
 // copies into and out of the split arrays (longer k runs per block; no
 // value depends on the split); kc: the SOR k chunk of the batch.
 void step_batch_spans(const DevDomain& d, int nzb, BatchDom* e, StageSpan* sp);
-void press_batch_spans(const DevDomain& d, int kc, int ty, int tw, int nzb, BatchDom* e, StageSpan* sp);
+void press_batch_spans(const DevDomain& d, bool res, int kc, int ty, int tw, int nzb, BatchDom* e, StageSpan* sp);
 // velnw .. les+adam of every domain, one launch per stage.
 void launch_step_batch(const StageBatch& b, hipStream_t stream);
 // part 0: rhs, its mean, the split arrays and SOR iteration 1; part 1 (after

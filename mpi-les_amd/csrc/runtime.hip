@@ -2000,6 +2000,11 @@ struct les_batch {
   // Domains whose whole step runs as batched stage launches (fused velfg and
   // les, batchable SOR); the others step on their own streams.
   std::vector<char> full;
+  // Those of them that solve in one launch, side by side (k_sor_res): the
+  // launches, their tables and their workspace.
+  std::vector<char> res;
+  std::vector<ResBatch> res_launch;
+  void* res_mem = nullptr;
   void* stage_mem = nullptr;      // device: BatchDom[nfull], then StageSpan[BS_N][nfull]
   StageBatch stages{};            // stages.nd == 0: no batched stages
   std::vector<DevDomain> key;     // domain states the table and graph were made for
@@ -2017,6 +2022,7 @@ void batch_free(les_batch* B) {
   if (B->gexec) hipGraphExecDestroy(B->gexec);
   dev_release(B->dtab);
   dev_release(B->stage_mem);
+  dev_release(B->res_mem);
   for (hipEvent_t e : B->head_done) hipEventDestroy(e);
   for (hipEvent_t e : B->tail_done) hipEventDestroy(e);
   if (B->fork) hipEventDestroy(B->fork);
@@ -2039,6 +2045,78 @@ bool batch_key_same(const les_batch* B) {
   return B->skey == batch_scalars(B);
 }
 
+// Cuts the domains that can solve in one launch for solving side by side, and
+// uploads their arguments.  One iteration of all domains per launch takes 8 us
+// (the launch) or 4.5 us per million cells; a batch whose solves are modelled
+// above that, many domains of which no two fit one kernel, keeps to it.
+int batch_res_prepare(les_batch* B) {
+  const size_t n = B->doms.size();
+  B->res.assign(n, 0);
+  B->res_launch.clear();
+  if (B->res_mem) {
+    HIP_TRY(hipStreamSynchronize(B->stream));
+    dev_release(B->res_mem);
+    B->res_mem = nullptr;
+  }
+  if (B->pairs || getenv("LES_BATCH_SOR_KCHUNK")) return 0;
+  std::vector<const DevDomain*> ds;
+  std::vector<int> at;
+  double cells = 0.0;
+  int ncu = 256;
+  for (size_t q = 0; q < n; q++) {
+    const DevDomain& d = B->doms[q]->d;
+    if (d.press_mode != 0 || !press_resident(d) || !d.fuse_velfg || !d.fuse_les) continue;
+    ds.push_back(&d);
+    at.push_back((int)q);
+    cells += (double)d.g.im * d.g.jm * d.g.km;
+    if (d.ncu > 0) ncu = d.ncu;
+  }
+  if (ds.empty()) return 0;
+  const int nd = (int)ds.size();
+  std::vector<ResShape> sh(nd);
+  std::vector<int> group;
+  const double us = res_batch_plan(ds.data(), nd, ncu, sh.data(), &group);
+  if (us < 0.0 || 2.0 * us > std::max(8.0, 4.5e-6 * cells)) return 0;
+  // arguments by launch, the launches' first blocks, then the workspaces
+  const int ng = 1 + *std::max_element(group.begin(), group.end());
+  std::vector<ResArgs> tab;
+  std::vector<int> b0s;
+  const size_t ntab = (nd * sizeof(ResArgs) + 255) / 256 * 256, nb0 = (nd * sizeof(int) + 255) / 256 * 256;
+  size_t words = 0;
+  for (int r = 0; r < nd; r++) words += (size_t)(res_words(ds[r]->g, ds[r]->sg, sh[r]) + 31) / 32 * 32;
+  HIP_TRY(dev_alloc(&B->res_mem, ntab + nb0 + 8 * words));
+  char* const base = (char*)B->res_mem;
+  unsigned long long* mem = (unsigned long long*)(base + ntab + nb0);
+  for (int q = 0; q < ng; q++) {
+    ResBatch L{};
+    L.tab = (const ResArgs*)base + tab.size();
+    L.b0 = (const int*)(base + ntab) + b0s.size();
+    L.om1 = true;
+    for (int r = 0; r < nd; r++) {
+      if (group[r] != q) continue;
+      const DevDomain& d = *ds[r];
+      SplitBufs sb = d.sb;
+      sb.cn1[0] = sb.cn1[1] = nullptr;  // separable cn1
+      tab.push_back(res_args(d, sh[r], mem, sb, d.nmaxp, d.pjuge, d.omega, false));
+      mem += (size_t)(res_words(d.g, d.sg, sh[r]) + 31) / 32 * 32;
+      b0s.push_back(L.blocks);
+      L.blocks += sh[r].nb + 1;
+      L.nd++;
+      L.cls = sh[r].cls;
+      L.nthr = sh[r].nthr;
+      L.kl = std::max(L.kl, sh[r].kl);
+      L.om1 = L.om1 && d.omega == 1.0f;
+      L.odd = L.odd || (d.g.im & 1) != 0;
+      B->res[at[r]] = 1;
+    }
+    B->res_launch.push_back(L);
+  }
+  HIP_TRY(hipMemsetAsync(base + ntab + nb0, 0, 8 * words, B->stream));
+  HIP_TRY(copy_sync(base, tab.data(), tab.size() * sizeof(ResArgs), hipMemcpyHostToDevice, B->stream));
+  HIP_TRY(copy_sync(base + ntab, b0s.data(), b0s.size() * sizeof(int), hipMemcpyHostToDevice, B->stream));
+  return 0;
+}
+
 // The SOR table and the stage tables for the domains' current states
 // (synchronous uploads).
 int batch_prepare(les_batch* B) {
@@ -2053,12 +2131,20 @@ int batch_prepare(les_batch* B) {
   std::vector<const DevDomain*> fd;
   long tiles = 0;  // (i,j) tiles of the stage kernels over the batched domains
   int ncu = 256;
+  for (les_domain* D : B->doms)
+    if (flush_metrics(D)) return 1;
+  // two iterations per launch measured no faster on batches of small domains
+  // (24 domains of 96..160 x 96..160 x 64: 8.0 against 8.1 ms per step, and
+  // 10.4 against 8.7 before tiles as wide as a domain lost their ring), so
+  // those that do not solve in one launch keep one iteration per launch unless
+  // LES_BATCH_SOR_PAIRS=1
+  B->pairs = env_int("LES_BATCH_SOR_PAIRS", 0) != 0;
+  if (batch_res_prepare(B)) return 1;
   for (size_t q = 0; q < B->doms.size(); q++) {
     les_domain* D = B->doms[q];
-    if (flush_metrics(D)) return 1;
-    if (!sor_batchable(D->d) || !D->d.fuse_velfg || !D->d.fuse_les) continue;
+    if ((!B->res[q] && !sor_batchable(D->d)) || !D->d.fuse_velfg || !D->d.fuse_les) continue;
     B->full[q] = 1;
-    fd.push_back(&D->d);
+    if (!B->res[q]) fd.push_back(&D->d);
     tiles += (long)((D->d.g.im + 63) / 64) * ((D->d.g.jm + 3) / 4);
     if (D->d.ncu > 0) ncu = D->d.ncu;
   }
@@ -2066,11 +2152,6 @@ int batch_prepare(les_batch* B) {
   // splits of the copy-like stages giving about 36 blocks per CU in all
   B->sor_ty = env_int("LES_BATCH_SOR_TILE_ROWS", 16) == 32 ? 32 : 16;
   B->sor_tw = (B->sor_ty == 32 && env_int("LES_BATCH_SOR_TILE_WIDTH", 64) == 32) ? 32 : 64;
-  // two iterations per launch measured no faster on batches of small domains
-  // (24 domains of 96..160 x 96..160 x 64: 8.0 against 8.1 ms per step, and
-  // 10.4 against 8.7 before tiles as wide as a domain lost their ring), so
-  // the batch keeps one iteration per launch unless LES_BATCH_SOR_PAIRS=1
-  B->pairs = env_int("LES_BATCH_SOR_PAIRS", 0) != 0;
   B->sor_kc = fd.empty() ? 0 : env_int("LES_BATCH_SOR_KCHUNK", 0);
   if (!fd.empty() && B->sor_kc <= 0)
     B->sor_kc = B->pairs ? sor_pair_batch_kchunk(fd.data(), (int)fd.size(), ncu)
@@ -2079,14 +2160,16 @@ int batch_prepare(les_batch* B) {
   for (size_t q = 0; q < B->doms.size(); q++) {
     if (!B->full[q]) continue;
     les_domain* D = B->doms[q];
-    SorBatchEntry e;
-    sor_batch_entry(D->d, B->sor_kc, B->sor_ty, B->sor_tw, &e, B->pairs);
-    e.block0 = block;
-    block += (e.nparts + 7) / 8 * 8;
-    B->kcmax = std::max(B->kcmax, e.kchunk);
-    B->lmax = std::max(B->lmax, e.nmaxp);
-    tab.push_back(e);
-    B->om1 = B->om1 && D->d.omega == 1.0f;
+    if (!B->res[q]) {
+      SorBatchEntry e;
+      sor_batch_entry(D->d, B->sor_kc, B->sor_ty, B->sor_tw, &e, B->pairs);
+      e.block0 = block;
+      block += (e.nparts + 7) / 8 * 8;
+      B->kcmax = std::max(B->kcmax, e.kchunk);
+      B->lmax = std::max(B->lmax, e.nmaxp);
+      tab.push_back(e);
+      B->om1 = B->om1 && D->d.omega == 1.0f;
+    }
     BatchDom bd{};
     std::array<StageSpan, BS_N> sp{};
     bd.d = D->d;
@@ -2096,7 +2179,7 @@ int batch_prepare(les_batch* B) {
     bd.alpha = D->alpha;
     bd.beta = D->beta;
     step_batch_spans(D->d, nzb, &bd, sp.data());
-    press_batch_spans(D->d, B->sor_kc, B->sor_ty, B->sor_tw, nzb, &bd, sp.data());
+    press_batch_spans(D->d, B->res[q] != 0, B->sor_kc, B->sor_ty, B->sor_tw, nzb, &bd, sp.data());
     bdom.push_back(bd);
     spans.push_back(sp);
   }
@@ -2120,6 +2203,8 @@ int batch_prepare(les_batch* B) {
     HIP_TRY(copy_sync(B->dtab, tab.data(), ntb, hipMemcpyHostToDevice, B->stream));
     HIP_TRY(copy_sync((char*)B->dtab + ntb, b0s.data(), b0s.size() * sizeof(int), hipMemcpyHostToDevice, B->stream));
     B->dblock0 = (const int*)((const char*)B->dtab + ntb);
+  }
+  if (!bdom.empty()) {
     // stage spans by stage, then domain; each domain's range of blocks starts
     // at a multiple of 8
     const int nd = (int)bdom.size();
@@ -2182,11 +2267,12 @@ int batch_enqueue(les_batch* B, const int* ns, const int* nmaxs, bool capturing)
       continue;
     }
     HIP_TRY(hipStreamWaitEvent(D->d.stream, B->fork, 0));
-    if (!B->full[q] && press_resident(D->d)) {  // those running the one-launch SOR step one after the other
+    // those running the one-launch SOR on their own step one after the other
+    if ((!B->full[q] || B->res[q]) && press_resident(D->d)) {
       if (res_prev >= 0) HIP_TRY(hipStreamWaitEvent(D->d.stream, B->head_done[res_prev], 0));
       res_prev = (int)q;
     }
-    if (B->full[q]) {
+    if (B->full[q] && !B->res[q]) {
       bool sp = false;
       if (run_step_head(D, ns[q], nmaxs[q], B->sor_kc, B->sor_ty, B->sor_tw, &sp)) return 1;
       split[q] = sp;
@@ -2199,6 +2285,7 @@ int batch_enqueue(les_batch* B, const int* ns, const int* nmaxs, bool capturing)
   if (staged) {
     launch_step_batch(B->stages, B->stream);
     launch_press_batch(B->stages, 0, B->stream);
+    for (const ResBatch& L : B->res_launch) launch_sor_res_batch(L, B->stream);
   }
   if (B->pairs && B->ntab > 0)
     launch_sor_pair_batch(B->dtab, B->dblock0, B->ntab, B->nblocks, B->lmax, B->kcmax, B->om1, B->remap, B->stream);
@@ -2288,8 +2375,9 @@ int les_batch_step(les_batch* B, const int* ns, const int* nmaxs) {
     if (flush_metrics(D)) return 1;  // synchronous: not under capture
     D->rhs_lazy = D->d.press_mode == 0;
   }
-  bool res = false;  // a domain stepping whole on its own stream runs the one-launch SOR
-  for (size_t q = 0; q < B->doms.size(); q++) res = res || (!B->full[q] && press_resident(B->doms[q]->d));
+  bool res = false;  // a domain runs the one-launch SOR, on its own stream or beside others
+  for (size_t q = 0; q < B->doms.size(); q++)
+    res = res || ((!B->full[q] || B->res[q]) && press_resident(B->doms[q]->d));
   ResOrder order(res, B->stream);
   HIP_TRY(order.err);
   bool replay = B->use_graph != 0;
