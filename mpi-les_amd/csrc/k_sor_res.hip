@@ -760,7 +760,8 @@ __device__ __forceinline__ void res_block(ConstArgs a0, const int bid) {
 // arguments are tab[e] and its blocks start at b0[e].  The domains of a batch
 // share the device side by side, each with boxes of its own and a handshake of
 // its own: 9 domains of 96..160 x 96..160 x 64 solve 50
-// iterations in 1165 us, one iteration of all of them per launch took 2090.
+// iterations in 880 us (two launches; 1165 in one, with boxes of 22 levels), one
+// iteration of all of them per launch took 2090.
 template <int CLS, int BK, bool OM1, bool ODD>
 __global__ __launch_bounds__(kResNT, 2 * kResClass[CLS].per) void k_sor_res(ResArgs a,
                                                                              const ResArgs* __restrict__ tab,
@@ -783,11 +784,15 @@ __global__ __launch_bounds__(kResNT, 2 * kResClass[CLS].per) void k_sor_res(ResA
 // Microseconds of one sweep of a cut, as a model: the sweep of a unit's boxes
 // (80 cycles per level and wave of a SIMD, no less than the latency of a wave
 // alone), the exchange (latency, and words per unit), and what a box of two
-// hides of it.  on: boxes on the fullest unit.
-static double res_cost(int waves, int kl, int nb, int words, int on) {
+// hides of it.  on: boxes on the fullest unit.  The tallest boxes of each class
+// spill registers: a sweep of 18 levels in class 1 takes 7.6 us at 300x300x90
+// where the rest of the model gives 5.4, one of 22 levels 11.6 for 6.0.
+static double res_cost(const ResShape& h, int words, int on) {
+  const int waves = h.nthr / kWave, kl = h.kl, over = kl - (h.cls == 0 ? 32 : 16);
+  const double slow = over <= 0 ? 1.0 : over <= 4 ? 1.4 : 2.0;
   const double sweep = std::max(0.034 * ((on * waves + 3) / 4), 0.055) * kl + 0.3 + 0.05 * waves * on;
-  const double cross = nb > 1 ? 1.5 + 0.35 * on * words / 1024 : 0.0;
-  return on == 1 ? sweep + cross : std::max(sweep, 0.6 * sweep + cross);
+  const double cross = h.nb > 1 ? 1.5 + 0.35 * on * words / 1024 : 0.0;
+  return slow * (on == 1 ? sweep + cross : std::max(sweep, 0.6 * sweep + cross));
 }
 
 static int up(int a, int b) { return (a + b - 1) / b; }
@@ -833,7 +838,7 @@ bool res_shape(const Grid& g, const SplitGrid& s, int units, ResShape* out) {
   double best = -1.0;
   for (int cls = 0; cls < 2; cls++)  // one block runs the monitor
     res_cuts(g, s, cls, kResClass[cls].per * units - 1, 0, kResClass[cls].levels, [&](const ResShape& h, int wds) {
-      const double c = res_cost(h.nthr / kWave, h.kl, h.nb, wds, h.nb > units ? 2 : 1);
+      const double c = res_cost(h, wds, h.nb > units ? 2 : 1);
       if (best < 0.0 || c < best) {
         best = c;
         *out = h;
@@ -863,7 +868,7 @@ static double res_batch_cut(const DevDomain* const* all, const std::vector<int>&
         const DevDomain& d = *all[ds[q]];
         std::vector<Cut> v;
         res_cuts(d.g, d.sg, cls, cap - 1, bk - 4, bk, [&](const ResShape& h, int wds) {
-          v.push_back({h, res_cost(h.nthr / kWave, h.kl, h.nb, wds, cls == 1 ? 2 : 1)});
+          v.push_back({h, res_cost(h, wds, cls == 1 ? 2 : 1)});
         });
         std::stable_sort(v.begin(), v.end(), [](const Cut& a, const Cut& b) { return a.h.nb < b.h.nb; });
         for (const Cut& c : v) {
@@ -909,12 +914,15 @@ double res_batch_plan(const DevDomain* const* ds, int n, int units, ResShape* sh
   for (int q = 0; q < n; q++) by[q] = q;
   const auto cells = [&](int q) { return (long)ds[q]->g.im * ds[q]->g.jm * ds[q]->g.km; };
   std::stable_sort(by.begin(), by.end(), [&](int a, int b) { return cells(a) > cells(b); });
+  // as few launches as hold them, or more while that is faster
+  double best = -1.0;
+  std::vector<ResShape> sh(n);
   for (int ng = 1; ng <= n; ng++) {
     std::vector<std::vector<int>> in(ng);  // dealt out there and back
     for (int r = 0; r < n; r++) in[(r / ng) & 1 ? ng - 1 - r % ng : r % ng].push_back(by[r]);
     double sum = 0.0;
     for (const auto& v : in) {
-      const double c = res_batch_cut(ds, v, units, shapes);
+      const double c = res_batch_cut(ds, v, units, sh.data());
       if (c < 0.0) {
         sum = -1.0;
         break;
@@ -922,12 +930,14 @@ double res_batch_plan(const DevDomain* const* ds, int n, int units, ResShape* sh
       sum += c;
     }
     if (sum < 0.0) continue;
+    if (best >= 0.0 && sum >= best) break;
+    best = sum;
+    std::copy(sh.begin(), sh.end(), shapes);
     group->assign(n, 0);
     for (int q = 0; q < ng; q++)
       for (int r : in[q]) (*group)[r] = q;
-    return sum;
   }
-  return -1.0;
+  return best;
 }
 
 // 8-byte words of the workspace: inboxes of both colours, the partial sums
