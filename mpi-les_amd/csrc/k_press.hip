@@ -1187,6 +1187,7 @@ struct PairLaunch {
   int gate;         // 0: runs; 1: runs only when no ghost of p differs from its boundp copy; 2: only when one does
   int prev_colours; // the previous launch ran one iteration in a one-iteration kernel (iteration 1 of a batch):
                     // its partials are sb.part[rpart][1] (red) and [0] (black) of that iteration
+  float c2, c3;     // cn2l = cn2s and cn3l = cn3s of a uniform grid (UNI)
 };
 
 // The stop test (press.f95:119-121) of a launch of iteration L (and L+1 when
@@ -1219,7 +1220,8 @@ constexpr int PTY = 32, PR = 4, PNT = FX * PTY / 2, PFTY = PTY - 2 * PR, PFTX = 
 
 // ENT: the launch may hold iteration 1 (the entry-ghost code is compiled in).
 // TW: 1 two iterations, 0 one (compiled in), -1 pl.two at run time (batches).
-template <bool OM1, bool ENT, int TW>
+// UNI: the grid is uniform in i and j (pl.c2, pl.c3; cn1 by level).
+template <bool OM1, bool ENT, int TW, bool UNI>
 __device__ __forceinline__ void sor_pair_block(const Grid& g, const SplitGrid& s, const Metrics& m,
                                                const SplitBufs& sb, Ctrl* ctrl, const PairLaunch& pl, int nparts,
                                                float omega, float pjuge, int ntt, int ntj, int kchunk, int remap,
@@ -1231,7 +1233,7 @@ __device__ __forceinline__ void sor_pair_block(const Grid& g, const SplitGrid& s
   __shared__ float ldsR2[2 * PL];  // C: red of l+1
   __shared__ double lds[GNT / kWave];
   __shared__ int sh[5];
-  extern __shared__ float4 lvm4[];  // per level from krs: cn4l, cn4s, cncz
+  extern __shared__ float4 lvm4[];  // per level from krs: cn4l, cn4s, cncz (UNI: cn1)
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.y);
   const int lane = (int)threadIdx.x;
   const int tid = w * FX + lane;
@@ -1305,15 +1307,18 @@ __device__ __forceinline__ void sor_pair_block(const Grid& g, const SplitGrid& s
   const bool wC = two && 2 * w + 1 >= 3 && 2 * w <= TY - 4;
   const bool wD = two && 2 * w + 1 >= 4 && 2 * w <= TY - 5;
   float c2l[2] = {0.f, 0.f}, c2s[2] = {0.f, 0.f}, axp[2] = {0.f, 0.f};
-  if (tin) {
+  if (UNI) {
+    c2l[0] = c2l[1] = c2s[0] = c2s[1] = pl.c2;
+  } else if (tin) {
     for (int p = 0; p < 2; p++) {
       c2l[p] = M1(m.cn2l, 2 * t + 1 + p);
       c2s[p] = M1(m.cn2s, 2 * t + 1 + p);
       axp[p] = M1(m.cnax, 2 * t + 1 + p);
     }
   }
-  const float c3lA = M1(m.cn3l, jA), c3sA = M1(m.cn3s, jA), c3lB = M1(m.cn3l, jB), c3sB = M1(m.cn3s, jB);
-  const float byA = M1(m.cnby, jA), byB = M1(m.cnby, jB);
+  const float c3lA = UNI ? pl.c3 : M1(m.cn3l, jA), c3sA = UNI ? pl.c3 : M1(m.cn3s, jA);
+  const float c3lB = UNI ? pl.c3 : M1(m.cn3l, jB), c3sB = UNI ? pl.c3 : M1(m.cn3s, jB);
+  const float byA = UNI ? 0.f : M1(m.cnby, jA), byB = UNI ? 0.f : M1(m.cnby, jB);
   float sA[2], sB[2];
   unsigned svA[2], svB[2];
   bool okA[2], okB[2], last[2];
@@ -1338,7 +1343,7 @@ __device__ __forceinline__ void sor_pair_block(const Grid& g, const SplitGrid& s
     if (k <= km) {
       v.x = M1(m.cn4l, k);
       v.y = M1(m.cn4s, k);
-      v.z = M1(m.cncz, k);
+      v.z = UNI ? m.lev4[4 * k + 2] : M1(m.cncz, k);
     }
     lvm4[x] = v;
   }
@@ -1364,6 +1369,9 @@ __device__ __forceinline__ void sor_pair_block(const Grid& g, const SplitGrid& s
   float rdA[3] = {0.f, 0.f, 0.f}, rdB[3] = {0.f, 0.f, 0.f};
   float blA[3] = {0.f, 0.f, 0.f}, blB[3] = {0.f, 0.f, 0.f};
   float r2A[3] = {0.f, 0.f, 0.f}, r2B[3] = {0.f, 0.f, 0.f};
+  // UNI: the rhs of A's and B's cells of the last three steps, for C and D two
+  // steps later (the registers of the per-column coefficients hold them)
+  float hrA3[3] = {0.f, 0.f, 0.f}, hrB3[3] = {0.f, 0.f, 0.f}, hbA3[3] = {0.f, 0.f, 0.f}, hbB3[3] = {0.f, 0.f, 0.f};
   // Level km+1 is the ghost boundp2 fills from level km: for A's red update
   // at km the cell itself, so that slot takes the red iterate of level km.
   const int lbq = min(aHi + 1, km + 1);
@@ -1405,11 +1413,21 @@ __device__ __forceinline__ void sor_pair_block(const Grid& g, const SplitGrid& s
       const bool actB = kb >= bLo && kb <= bHi;
       const bool actC = two && kc >= cLo && kc <= cHi;
       const bool actD = two && kd >= k0 && kd <= k1;
-      // 1. the rhs of C's and D's cells, read again (the lines were read two
+      // 1. the rhs of C's and D's cells, kept (UNI) or read again (the lines were read two
       // steps earlier for A and B, so they come from the caches), and the
       // black iterate of l-1 at level kr+1 into its plane
       float hrA = 0.f, hrB = 0.f, hbA = 0.f, hbB = 0.f;
-      if (two) {
+      if (UNI) {
+        const Sl& q0 = sl[U % 2];
+        hrA3[U % 3] = q0.rrA;
+        hrB3[U % 3] = q0.rrB;
+        hbA3[U % 3] = q0.rbA;
+        hbB3[U % 3] = q0.rbB;
+        hrA = hrA3[(U + 1) % 3];
+        hrB = hrB3[(U + 1) % 3];
+        hbA = hbA3[(U + 1) % 3];
+        hbB = hbB3[(U + 1) % 3];
+      } else if (two) {
         const unsigned lc = (unsigned)min(max(kc, 1), km) * cplb, ld = (unsigned)min(max(kd, 1), km) * cplb;
         hrA = bload(S, voA, orR + lc);
         hrB = bload(S, voB, orR + lc);
@@ -1444,7 +1462,7 @@ __device__ __forceinline__ void sor_pair_block(const Grid& g, const SplitGrid& s
             if (kr == 1) pkm = pent[ix(g, i, jA, 0)];
             if (kr == km) pkp = pent[ix(g, i, jA, km + 1)];
           }
-          const float cn = rcp_rn(sA[pa] + mt.z);  // init.f95:100-107
+          const float cn = UNI ? mt.z : rcp_rn(sA[pa] + mt.z);  // init.f95:100-107
           const float reltmp = relax<OM1>(omega, cn * (c2l[pa] * pip + c2s[pa] * pim + c3lA * pjp + c3sA * pjm +
                                                        mt.x * pkp + mt.y * pkm - q.rrA) -
                                                      own);
@@ -1470,7 +1488,7 @@ __device__ __forceinline__ void sor_pair_block(const Grid& g, const SplitGrid& s
             if (kr == 1) pkm = pent[ix(g, i, jB, 0)];
             if (kr == km) pkp = pent[ix(g, i, jB, km + 1)];
           }
-          const float cn = rcp_rn(sB[pb] + mt.z);
+          const float cn = UNI ? mt.z : rcp_rn(sB[pb] + mt.z);
           const float reltmp = relax<OM1>(omega, cn * (c2l[pb] * pip + c2s[pb] * pim + c3lB * pjp + c3sB * pjm +
                                                        mt.x * pkp + mt.y * pkm - q.rrB) -
                                                      own);
@@ -1504,7 +1522,7 @@ __device__ __forceinline__ void sor_pair_block(const Grid& g, const SplitGrid& s
             if (kb == 1) pkm = pent[ix(g, i, jA, 0)];
             if (kb == km) pkp = pent[ix(g, i, jA, km + 1)];
           }
-          const float cn = rcp_rn(sA[pa] + mt.z);
+          const float cn = UNI ? mt.z : rcp_rn(sA[pa] + mt.z);
           const float reltmp = relax<OM1>(omega, cn * (c2l[pa] * pip + c2s[pa] * pim + c3lA * pjp + c3sA * pjm +
                                                        mt.x * pkp + mt.y * pkm - q.rbA) -
                                                      own);
@@ -1526,7 +1544,7 @@ __device__ __forceinline__ void sor_pair_block(const Grid& g, const SplitGrid& s
             if (kb == 1) pkm = pent[ix(g, i, jB, 0)];
             if (kb == km) pkp = pent[ix(g, i, jB, km + 1)];
           }
-          const float cn = rcp_rn(sB[pb] + mt.z);
+          const float cn = UNI ? mt.z : rcp_rn(sB[pb] + mt.z);
           const float reltmp = relax<OM1>(omega, cn * (c2l[pb] * pip + c2s[pb] * pim + c3lB * pjp + c3sB * pjm +
                                                        mt.x * pkp + mt.y * pkm - q.rbB) -
                                                      own);
@@ -1555,7 +1573,7 @@ __device__ __forceinline__ void sor_pair_block(const Grid& g, const SplitGrid& s
           const float pjp = blB[(U + 1) % 3];
           const float pkm = (kc == 1) ? own : blA[U % 3];
           const float pkp = (kc == km) ? own : blA[(U + 2) % 3];
-          const float cn = rcp_rn(sA[pa] + mt.z);
+          const float cn = UNI ? mt.z : rcp_rn(sA[pa] + mt.z);
           const float reltmp = relax<OM1>(omega, cn * (c2l[pa] * pip + c2s[pa] * pim + c3lA * pjp + c3sA * pjm +
                                                        mt.x * pkp + mt.y * pkm - hrA) -
                                                      own);
@@ -1572,7 +1590,7 @@ __device__ __forceinline__ void sor_pair_block(const Grid& g, const SplitGrid& s
           const float pjp = pq[dnB];
           const float pkm = (kc == 1) ? own : blB[U % 3];
           const float pkp = (kc == km) ? own : blB[(U + 2) % 3];
-          const float cn = rcp_rn(sB[pb] + mt.z);
+          const float cn = UNI ? mt.z : rcp_rn(sB[pb] + mt.z);
           const float reltmp = relax<OM1>(omega, cn * (c2l[pb] * pip + c2s[pb] * pim + c3lB * pjp + c3sB * pjm +
                                                        mt.x * pkp + mt.y * pkm - hrB) -
                                                      own);
@@ -1599,7 +1617,7 @@ __device__ __forceinline__ void sor_pair_block(const Grid& g, const SplitGrid& s
           const float pjp = r2B[U % 3];
           const float pkm = (kd == 1) ? own : r2A[(U + 2) % 3];
           const float pkp = (kd == km) ? own : r2a;
-          const float cn = rcp_rn(sA[pa] + mt.z);
+          const float cn = UNI ? mt.z : rcp_rn(sA[pa] + mt.z);
           const float reltmp = relax<OM1>(omega, cn * (c2l[pa] * pip + c2s[pa] * pim + c3lA * pjp + c3sA * pjm +
                                                        mt.x * pkp + mt.y * pkm - hbA) -
                                                      own);
@@ -1615,7 +1633,7 @@ __device__ __forceinline__ void sor_pair_block(const Grid& g, const SplitGrid& s
           const float pjp = pr[dnB];
           const float pkm = (kd == 1) ? own : r2B[(U + 2) % 3];
           const float pkp = (kd == km) ? own : r2b;
-          const float cn = rcp_rn(sB[pb] + mt.z);
+          const float cn = UNI ? mt.z : rcp_rn(sB[pb] + mt.z);
           const float reltmp = relax<OM1>(omega, cn * (c2l[pb] * pip + c2s[pb] * pim + c3lB * pjp + c3sB * pjm +
                                                        mt.x * pkp + mt.y * pkm - hbB) -
                                                      own);
@@ -1662,11 +1680,11 @@ __device__ __forceinline__ void sor_pair_block(const Grid& g, const SplitGrid& s
   }
 }
 
-template <bool OM1, bool ENT, int TW>
+template <bool OM1, bool ENT, int TW, bool UNI>
 __global__ __launch_bounds__(PNT) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_sor_pair(
     Grid g, SplitGrid s, Metrics m, SplitBufs sb, Ctrl* ctrl, PairLaunch pl, int nparts, float omega, float pjuge,
     int ntt, int ntj, int kchunk, int remap, const float* __restrict__ pent) {
-  sor_pair_block<OM1, ENT, TW>(g, s, m, sb, ctrl, pl, nparts, omega, pjuge, ntt, ntj, kchunk, remap, pent,
+  sor_pair_block<OM1, ENT, TW, UNI>(g, s, m, sb, ctrl, pl, nparts, omega, pjuge, ntt, ntj, kchunk, remap, pent,
                            (int)blockIdx.x);
 }
 
@@ -1707,7 +1725,7 @@ __global__ __launch_bounds__(PNT) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
     pl.two = pl.two && pl.iter + 1 <= E.nmaxp;
     pl.prev_nparts = pl.prev_colours ? E.nparts1 : E.nparts;
   }
-  sor_pair_block<OM1, false, -1>(E.g, E.s, E.m, E.sb, E.ctrl, pl, E.nparts, E.omega, E.pjuge, E.ntt, E.ntj, E.kchunk,
+  sor_pair_block<OM1, false, -1, false>(E.g, E.s, E.m, E.sb, E.ctrl, pl, E.nparts, E.omega, E.pjuge, E.ntt, E.ntj, E.kchunk,
                              remap, nullptr, bid);
 }
 
@@ -2071,34 +2089,48 @@ static SorShape sor_shape_single(const DevDomain& d) {
                    d.sor_tile_width);
 }
 
-// One launch of k_sor_pair (two iterations, one, or the fix-up).
-static void launch_pair(const DevDomain& d, const SplitBufs& sb, const PairLaunch& pl, const SorShape& h, float pjuge,
+// One launch of k_sor_pair (two iterations, one, or the fix-up).  A grid
+// uniform in i and j takes the kernel without the per-column coefficients and
+// their reciprocals (4 of 22 vector instructions per update), whose registers
+// keep the right-hand sides that C and D would read again (4 of 16 memory
+// instructions per step).  160 us before, 132 now per launch at 512x512x128;
+// 612 and 505 at 1024x1024x128.  Not where the entry-ghost code is compiled in
+// (one or two launches per press): that kernel spills already.
+static void launch_pair(const DevDomain& d, const SplitBufs& sb, const PairLaunch& pl0, const SorShape& h, float pjuge,
                         const float* pent) {
   const size_t lvm_bytes = (size_t)(h.kc + 7) * sizeof(float4);
+  PairLaunch pl = pl0;
+  pl.c2 = d.res_c2;
+  pl.c3 = d.res_c3;
   const bool ent = (pl.iter == 1 || pl.fixup) && pent;  // may run iteration 1 on the entry ghosts
+  const bool uni = !ent && d.res_uniform;
   const int cls = (pl.iter == 1 || pl.fixup) ? KC_SOR1 : KC_SOR;
   const bool two = pl.two != 0 && !pl.fixup;  // compiled in: no branch on it in the march
-#define PAIR1(OM1, ENT, TW)                                                                                     \
-  TIMED(d, cls, hipLaunchKernelGGL((k_sor_pair<OM1, ENT, TW>), dim3(h.nparts), dim3(FX, PTY / 2), lvm_bytes,       \
+#define PAIR1(OM1, ENT, TW, UNI)                                                                                \
+  TIMED(d, cls, hipLaunchKernelGGL((k_sor_pair<OM1, ENT, TW, UNI>), dim3(h.nparts), dim3(FX, PTY / 2), lvm_bytes,  \
                                    d.stream, d.g, d.sg, d.m, sb, d.ctrl, pl, h.nparts, d.omega, pjuge, h.ntt,      \
                                    h.ntj, h.kc, d.xcd_remap, pent))
-#define PAIR(OM1, ENT)       \
-  do {                       \
-    if (two)                 \
-      PAIR1(OM1, ENT, 1);    \
-    else                     \
-      PAIR1(OM1, ENT, 0);    \
+#define PAIR(OM1, ENT, UNI)       \
+  do {                            \
+    if (two)                      \
+      PAIR1(OM1, ENT, 1, UNI);    \
+    else                          \
+      PAIR1(OM1, ENT, 0, UNI);    \
   } while (0)
   if (d.omega == 1.0f) {
     if (ent)
-      PAIR(true, true);
+      PAIR(true, true, false);
+    else if (uni)
+      PAIR(true, false, true);
     else
-      PAIR(true, false);
+      PAIR(true, false, false);
   } else {
     if (ent)
-      PAIR(false, true);
+      PAIR(false, true, false);
+    else if (uni)
+      PAIR(false, false, true);
     else
-      PAIR(false, false);
+      PAIR(false, false, false);
   }
 #undef PAIR
 #undef PAIR1

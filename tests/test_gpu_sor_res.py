@@ -188,3 +188,22 @@ def test_inner_solves_of_the_defect_correction(dims, outer, inner, omega, mode):
         assert outer != 6 or n > 1 or st["iters"] == 4, st["iters"]
     ref.close()
     res.close()
+
+
+@pytest.mark.parametrize("dims", [(130, 50, 12), (121, 14, 17)], ids=["even", "odd im"])
+def test_two_iterations_per_launch_on_either_grid(dims):
+    """k_sor_pair with and without per-column coefficients against one
+    iteration per launch."""
+    s = setup_gen.build(setup_gen.small_workload(*dims, seed=9), dense=False)
+    c = dict(s.coeffs, cn2l=s.coeffs["cn2l"].copy(), cn3s=s.coeffs["cn3s"].copy())
+    c["cn2l"][5] *= np.float32(1.25)
+    c["cn3s"][3] *= np.float32(0.75)
+    for q, grid in enumerate((s, dataclasses.replace(s, coeffs=c))):
+        print(f"\n[sor pair grid] {dims} {q}", flush=True)
+        a, b = _domain(grid, LES_SOR_ROWS=2), _domain(grid, LES_SOR_ROWS=4)
+        for n in (1, 2, 3):
+            a.step(n, 3)
+            b.step(n, 3)
+            _same(a, b, n)
+        a.close()
+        b.close()
