@@ -204,6 +204,7 @@ __global__ __launch_bounds__(NT) void k_rhs_head(Grid g, SplitGrid s, Metrics m,
     ctrl->nonfinite = 0;
     ctrl->p_final = -1;
     ctrl->fix_iter = 0;
+    res_begin(ctrl);  // the solve may run in one launch
   }
   const int i = 1 + vb.x * BX + threadIdx.x, j = 1 + vb.y * BY + wave_row();
   double acc = 0.0;
@@ -306,7 +307,6 @@ __global__ __launch_bounds__(256) void k_finalize_head(const double* __restrict_
   if (threadIdx.x == 0) {
     ctrl->rhsav = s / denom;
     ctrl->p_ghost_diff = fl != 0.0 ? 1 : 0;
-    res_begin(ctrl);
   }
 }
 
@@ -2569,16 +2569,16 @@ void launch_press(const DevDomain& d, float dt) {
     TIMED(d, KC_RHS, hipLaunchKernelGGL(k_rhs_head, dim3(gx, gy, gz), blk(), 0, d.stream, g, s, d.m,
                                         (const float*)d.F.u, (const float*)d.F.v, (const float*)d.F.w, d.F.f,
                                         d.F.g, d.F.h, (const float*)d.F.p, sb, d.partials, nred, d.ctrl, dt));
+    if (res) {  // the whole solve in one launch, the mean removal included
+      launch_sor_res(d, sb, d.nmaxp, d.pjuge, d.omega, false, nred);
+      launch_press_mean(d, sb, gx, gy, gz, nred);
+      return;
+    }
     TIMED(d, KC_RHS, hipLaunchKernelGGL(k_finalize_head, dim3(1), dim3(256), 0, d.stream,
                                         (const double*)d.partials, nred, d.ctrl, d.area));
     const long n4 = (long)s.cplane * g.km / 2;  // both colours, four floats at a time
     TIMED(d, KC_RHS, hipLaunchKernelGGL(k_rhs_sub, dim3(kRhsSubBlocks), dim3(256), 0, d.stream,
                                         (const float4*)sb.rhsr[0], (float4*)sb.rhs[0], n4, (const Ctrl*)d.ctrl));
-    if (res) {  // the whole solve in one launch
-      launch_sor_res(d, sb, d.nmaxp, d.pjuge, d.omega, false);
-      launch_press_mean(d, sb, gx, gy, gz, nred);
-      return;
-    }
     const PairLaunch last = launch_sor_pairs(d, sb, h, d.pjuge, 1, d.nmaxp, 0, d.F.p);
     TIMED(d, KC_PAV, hipLaunchKernelGGL(k_sor_pair_final, dim3(1), dim3(256), 0, d.stream, sb, d.ctrl, last,
                                         h.nparts, d.pjuge));

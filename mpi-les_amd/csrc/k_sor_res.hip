@@ -23,10 +23,10 @@
 // useful at 300x300x90).  Microseconds of a 50-iteration solve, before and
 // now: 24x20x16 455 and 196, 96x96x64 498 and 242, 150x150x90 675 and 341,
 // 203x117x61 878 and 329 (odd jm: one iteration per launch before), 300x300x90
-// 1130 and 790.
+// 1130 and 680.
 //
 // Waiting on other blocks is safe only while all of them run.  The blocks
-// first count themselves in (res_enter).  When all have arrived, none can be
+// first count themselves in (res_arrive, res_enter).  When all have arrived, none can be
 // left unscheduled and the waits always end.  When they have not within
 // kEnterTicks (another process's blocks hold the compute units), the launch
 // falls back to sweeps over memory handed out by a ticket counter
@@ -121,6 +121,24 @@ __device__ __forceinline__ double res_block_sum(double v, int tid, int nthr, dou
   return s;
 }
 
+// The mean of the rhs, in every thread: the partial sums added in the order of
+// k_finalize_head's 256 threads.
+__device__ __forceinline__ double res_mean(ConstArgs a, int tid, int nthr, double* lds) {
+  const int n = a->nred, lane = tid % kWave;
+  const double* const part = a->rpart;
+  for (int w = tid / kWave; w < 256 / kWave; w += nthr / kWave) {
+    double s = 0.0;
+    for (int b = w * kWave + lane; b < n; b += 256) s += part[b];
+    for (int o = kWave / 2; o > 0; o >>= 1) s += __shfl_xor(s, o, kWave);
+    if (lane == 0) lds[w] = s;
+  }
+  __syncthreads();
+  double s = 0.0;
+  for (int w = 0; w < 256 / kWave; w++) s += lds[w];
+  __syncthreads();
+  return s / a->area;
+}
+
 // Records iteration l's sum of reltmp^2 and returns whether it stops the
 // loop (press.f95:119-121, or a non-finite sum).
 __device__ __forceinline__ bool res_record(Ctrl* ctrl, int l, double s, float pjuge, bool writer) {
@@ -185,15 +203,15 @@ __device__ __forceinline__ int res_verdict(ConstArgs a, int np, int l, unsigned 
 // runs by tickets.  Thread 0 of each block; the last block to arrive decides
 // 1, a block that waited kEnterTicks (or force_ticket) decides 2, whichever
 // comes first.
-__device__ __forceinline__ int res_enter(Ctrl* ctrl, int nb, int force_ticket) {
-  if (force_ticket) return 2;
+__device__ __forceinline__ void res_arrive(Ctrl* ctrl, int nb) {
   const int n = __hip_atomic_fetch_add(&ctrl->res_arrived, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   if (n == nb - 1) {
     int want = 0;
     __hip_atomic_compare_exchange_strong(&ctrl->res_state, &want, 1, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
                                          __HIP_MEMORY_SCOPE_AGENT);
-    return ald(&ctrl->res_state);
   }
+}
+__device__ __forceinline__ int res_enter(Ctrl* ctrl) {
   const long long t0 = wall_clock64();
   for (;;) {
     const int st = ald(&ctrl->res_state);
@@ -212,7 +230,7 @@ __device__ __forceinline__ int res_enter(Ctrl* ctrl, int nb, int force_ticket) {
 // and 1 by iteration parity, as k_sweep), each cut into tickets taken in
 // order.  A sweep starts when the one before is complete; its tickets were
 // taken before and are held by running blocks.
-__device__ __forceinline__ void res_ticket(ConstArgs a0, float* lds_f) {
+__device__ __forceinline__ void res_ticket(ConstArgs a0, float* lds_f, double av) {
   double* const lds = (double*)lds_f;
   int* const sh = (int*)(lds_f + 2 * (kResNT / kWave));
   const int tid = threadIdx.x, nthr = blockDim.x;
@@ -221,6 +239,7 @@ __device__ __forceinline__ void res_ticket(ConstArgs a0, float* lds_f) {
   const SplitGrid s = {a->s.nt, a->s.cp, a->s.cplane};
   Ctrl* ctrl = a->ctrl;
   const int im = g.im, jm = g.jm, km = g.km, nt = s.nt;
+  if (a->nred > 0 && blockIdx.x == 0 && tid == 0) ctrl->rhsav = av;
   const int npr = nt * jm;                          // pairs per level
   const int chunks = (npr + nthr - 1) / nthr;      // tickets per level
   const int per = chunks * km;                      // tickets per sweep
@@ -260,6 +279,7 @@ __device__ __forceinline__ void res_ticket(ConstArgs a0, float* lds_f) {
         for (int c = 0; c < 2; c++) {
           const int i = 2 * t + 1 + ((1 + j + k + c) & 1);
           a->sb.p[0][c][q] = (a->zero || i > im) ? 0.0f : a->pent[ix(g, i, j, k)];
+          if (a->nred > 0) a->sb.rhs[c][q] = (float)((double)a->rhsr[c][q] - av);
         }
       } else {
         const int pos = (1 + j + k + col) & 1, i = 2 * t + 1 + pos;
@@ -338,20 +358,24 @@ __device__ __forceinline__ void res_block(ConstArgs a0, const int bid) {
   constexpr int NG = (BK + G - 1) / G, NT = kResNT, RL = res_lds_rhs(CLS, BK);
   __shared__ float S[BK * PLANE];
   __shared__ float RB[RL > 0 ? RL * NT : 1];  // rhs of the black cells of levels below RL, by thread
-  __shared__ double wsum[NT / kWave];
+  __shared__ double wsum[NT / kWave], av_s;
   __shared__ int sh[3];  // mode; a wait that gave up; the monitor's verdict
   const int tid = threadIdx.x, nthr = blockDim.x, nwav = nthr / kWave;
   const int nb = a0->nb;
+  // sor_done set on entry (a finished defect correction): nothing to solve
+  const bool skip = a0->ctrl->sor_done != 0;  // (no block passes res_enter, to change it, before all have read it)
+  if (tid == 0 && !skip && !a0->force_ticket) res_arrive(a0->ctrl, nb + 1);
+  const double av = a0->nred > 0 ? res_mean(again(a0), tid, nthr, wsum) : 0.0;  // while the others arrive
   if (tid == 0) {
-    // sor_done set on entry (a finished defect correction): nothing to solve
-    sh[0] = a0->ctrl->sor_done != 0 ? 0 : res_enter(a0->ctrl, nb + 1, a0->force_ticket);
+    sh[0] = skip ? 0 : a0->force_ticket ? 2 : res_enter(a0->ctrl);
     sh[1] = 0;
+    av_s = av;  // read where the rhs is
   }
   __syncthreads();
   const int mode = sh[0];
   if (mode == 0) return;
   if (mode == 2) {
-    res_ticket(a0, S);
+    res_ticket(a0, S, av);
     return;
   }
   if (bid == nb) {
@@ -463,18 +487,34 @@ __device__ __forceinline__ void res_block(ConstArgs a0, const int bid) {
       const int j0 = 1 + by * g.jm / a->nty, tjn = (by + 1) * g.jm / a->nty + 1 - j0;
       const int tg = t0 + ce % W - 1, j = j0 + ce / W - 1;
       {
-        const float* r0 = a->sb.rhs[0] + rcix(s, tg, j, k0);
-        const float* r1 = a->sb.rhs[1] + rcix(s, tg, j, k0);
+        const bool mean = a->nred > 0;
+        const double av = av_s;
+        const int rq = rcix(s, tg, j, k0);
+        const float* r0 = (mean ? a->rhsr[0] : a->sb.rhs[0]) + rq;
+        const float* r1 = (mean ? a->rhsr[1] : a->sb.rhs[1]) + rq;
+        float* w0 = a->sb.rhs[0] + rq;
+        float* w1 = a->sb.rhs[1] + rq;
         const float* pp = pent + ix(g, 2 * tg + 1, j, k0);  // i = 1 is 256-byte aligned
 #pragma unroll
         for (int kk = 0; kk < BK; kk++) {
           v[0][kk] = v[1][kk] = rh[0][kk] = rh[1][kk] = 0.0f;
           if (kk < BK - 4 || kk < nlev) {
+            float x0 = *r0, x1 = *r1;
+            if (mean) {  // press.f95:81-87, the subtraction in FP64 as in k_rhs_sub
+              x0 = (float)((double)x0 - av);
+              x1 = (float)((double)x1 - av);
+              if (act) {
+                *w0 = x0;
+                *w1 = x1;
+              }
+              w0 += s.cplane;
+              w1 += s.cplane;
+            }
             if (kk < RL)
-              RB[kk * NT + tid] = *r0;
+              RB[kk * NT + tid] = x0;
             else
-              rh[0][kk] = *r0;
-            rh[1][kk] = *r1;
+              rh[0][kk] = x0;
+            rh[1][kk] = x1;
             if (!zero) {
               const float2 x = *(const float2*)pp;
               const bool pr = (side > 0) != ((kk & 1) != 0);  // red at position 1
@@ -752,7 +792,10 @@ __device__ __forceinline__ void res_block(ConstArgs a0, const int bid) {
           r[kk * cpl] = v[1][kk];
         }
     }
-    if (writer) a->ctrl->p_final = 1;
+    if (writer) {
+      a->ctrl->p_final = 1;
+      if (a->nred > 0) a->ctrl->rhsav = av_s;
+    }
   }
 }
 
@@ -785,11 +828,11 @@ __global__ __launch_bounds__(kResNT, 2 * kResClass[CLS].per) void k_sor_res(ResA
 // (80 cycles per level and wave of a SIMD, no less than the latency of a wave
 // alone), the exchange (latency, and words per unit), and what a box of two
 // hides of it.  on: boxes on the fullest unit.  The tallest boxes of each class
-// spill registers: a sweep of 18 levels in class 1 takes 7.6 us at 300x300x90
-// where the rest of the model gives 5.4, one of 22 levels 11.6 for 6.0.
+// spill registers: a sweep of 18 levels in class 1 takes 6.8 us at 300x300x90
+// where the rest of the model gives 5.4, one of 22 levels 9.7 for 6.0.
 static double res_cost(const ResShape& h, int words, int on) {
   const int waves = h.nthr / kWave, kl = h.kl, over = kl - (h.cls == 0 ? 32 : 16);
-  const double slow = over <= 0 ? 1.0 : over <= 4 ? 1.4 : 2.0;
+  const double slow = over <= 0 ? 1.0 : over <= 2 ? 1.25 : over <= 4 ? 1.4 : over <= 6 ? 1.65 : 2.0;
   const double sweep = std::max(0.034 * ((on * waves + 3) / 4), 0.055) * kl + 0.3 + 0.05 * waves * on;
   const double cross = h.nb > 1 ? 1.5 + 0.35 * on * words / 1024 : 0.0;
   return slow * (on == 1 ? sweep + cross : std::max(sweep, 0.6 * sweep + cross));
@@ -1001,7 +1044,11 @@ static void launch_res(const ResGrid& r, const ResArgs& a) {
   RES(8)
   RES(12)
   RES(16)
+  // (every two levels where registers spill: 300x300x90, boxes of 18 levels,
+  // takes 680 us per solve, in the kernel for 20 levels 760)
+  if constexpr (CLS == 1) RES(18)
   RES(20)
+  if constexpr (CLS == 1) RES(22)
   RES(24)
   if constexpr (CLS == 0) {
     RES(28)
@@ -1030,9 +1077,15 @@ static void launch_res(const ResGrid& r, const ResArgs& a, int cls, bool om1, bo
   }
 }
 
-void launch_sor_res(const DevDomain& d, const SplitBufs& sb, int nmaxp, float pjuge, float omega, bool zero) {
+void launch_sor_res(const DevDomain& d, const SplitBufs& sb, int nmaxp, float pjuge, float omega, bool zero,
+                    int nred) {
   const ResShape& h = d.res;
-  const ResArgs a = res_args(d, h, d.res_mem, sb, nmaxp, pjuge, omega, zero);
+  ResArgs a = res_args(d, h, d.res_mem, sb, nmaxp, pjuge, omega, zero);
+  a.rhsr[0] = sb.rhsr[0];
+  a.rhsr[1] = sb.rhsr[1];
+  a.rpart = d.partials;
+  a.nred = nred;
+  a.area = d.area;
   const ResGrid r{h.nb + 1, h.nthr, h.kl, d.stream, nullptr, nullptr, 0};
   TIMED(d, KC_SOR, launch_res(r, a, h.cls, omega == 1.0f, (d.g.im & 1) != 0));
 }

@@ -54,6 +54,10 @@ struct ResArgs {
   Metrics m;
   SplitBufs sb;                // reads rhs, writes iterate set 1
   Ctrl* ctrl;
+  const float* rhsr[2];        // the rhs before its mean is removed (nullptr: sb.rhs is final) ...
+  const double* rpart;         // ... whose mean is the sum of nred partial sums over area
+  int nred;
+  double area;
   const float* pent;           // the padded field p: start iterate and the ghosts it had on entry
   unsigned long long* slots;   // halo words: inboxes of the black, then of the red cells
   unsigned long long* parts;   // partial sums of four iterations, two words each
@@ -133,7 +137,10 @@ inline bool press_resident(const DevDomain& d) {
   return use_res(d) && (d.press_mode == 0 ? d.nmaxp : d.dc_inner) >= 1;
 }
 // One solve: from the field p and its ghosts (zero: from 0) to iterate set 1.
-void launch_sor_res(const DevDomain& d, const SplitBufs& sb, int nmaxp, float pjuge, float omega, bool zero);
+// nred > 0: of the rhs in sb.rhsr, whose mean (from the partial sums
+// d.partials) it removes.
+void launch_sor_res(const DevDomain& d, const SplitBufs& sb, int nmaxp, float pjuge, float omega, bool zero,
+                    int nred = 0);
 // The same for a batch of domains, in one launch per group: group[q] and
 // shapes[q] of domain q.  Returns the modelled microseconds per colour sweep
 // of all of them, negative when one fits no cut.
