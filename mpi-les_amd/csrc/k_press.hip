@@ -2245,7 +2245,7 @@ static void launch_press_dc(const DevDomain& d, const SplitBufs& sb, int gx, int
   // SOR runs so (iterate sets rotating over three from set 0, which
   // k_dc_defect clears), else one per launch; they never stop on their own
   // (threshold 0).  16 steps at 256x256x64 with the iterations two per launch
-  // take 47.1 ms, in one launch per inner solve 36.6.
+  // take 47.1 ms, in one launch per inner solve 26.5.
   const SorShape hp = sor_shape(d);
   const bool res = press_resident(d), pairs = hp.rows == 4;
   const SorShape h = pairs ? hp : sor_shape_single(d);

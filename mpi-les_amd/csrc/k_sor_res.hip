@@ -21,9 +21,9 @@
 // cost 8 us each on the smallest domains and recompute a four-cell ring and
 // six extra levels per block on large ones (0.37 of their lane-steps are
 // useful at 300x300x90).  Microseconds of a 50-iteration solve, before and
-// now: 24x20x16 455 and 196, 96x96x64 498 and 242, 150x150x90 675 and 341,
-// 203x117x61 878 and 329 (odd jm: one iteration per launch before), 300x300x90
-// 1130 and 680.
+// now: 24x20x16 455 and 163, 96x96x64 498 and 232, 150x150x90 675 and 319,
+// 203x117x61 878 and 318 (odd jm: one iteration per launch before), 256x256x64
+// 898 and 385, 300x300x90 1130 and 658.
 //
 // Waiting on other blocks is safe only while all of them run.  The blocks
 // first count themselves in (res_arrive, res_enter).  When all have arrived, none can be
@@ -711,7 +711,12 @@ __device__ __forceinline__ void res_block(ConstArgs a0, const int bid) {
             ast(pw + 1, wq | (bits & 0xffffffffull));
           }
         }
-        // ---- receive the halo
+        // ---- receive the halo, and the verdict on iteration l-2, published
+        // during l-1 (asked for first: a look of its own takes as long as the
+        // exchange, 677 us instead of 657 per solve at 300x300x90)
+        const bool ask = c == 0 && pass == 0 && l > 2 && tid == 0;
+        u64 said = 0;
+        if (ask) said = ald(a->parts + 8 * (size_t)(nb * nwav) + ((l - 2) & 3));
         if (nb > 1) {
           const u64* const me = inb + (unsigned)(bid * a->iw);
           u64 w[NW], wk[2] = {0, 0};
@@ -739,10 +744,9 @@ __device__ __forceinline__ void res_block(ConstArgs a0, const int bid) {
           for (int q = 0; q < NW; q++)
             if (q < nqo) S[(wsd[q] >> 16) + ((wto[q] >> 31) ? cw : 0)] = wval(w[q]);
         }
-        {
-          // the verdict on iteration l-2, published during l-1
-          if (c == 0 && pass == 0 && l > 2 && tid == 0)
-            sh[2] = res_verdict(a, nb * nwav, l - 2, tag + 2 * (l - 2), &sh[1]);
+        if (ask) {
+          const unsigned pt = tag + 2 * (l - 2);
+          sh[2] = wtag(said) == pt ? (int)(said & 1u) : res_verdict(a, nb * nwav, l - 2, pt, &sh[1]);
         }
         __syncthreads();  // the halo is in place
         if (sh[1]) {
@@ -829,13 +833,17 @@ __global__ __launch_bounds__(kResNT, 2 * kResClass[CLS].per) void k_sor_res(ResA
 // alone), the exchange (latency, and words per unit), and what a box of two
 // hides of it.  on: boxes on the fullest unit.  The tallest boxes of each class
 // spill registers: a sweep of 18 levels in class 1 takes 6.8 us at 300x300x90
-// where the rest of the model gives 5.4, one of 22 levels 9.7 for 6.0.
+// where the rest of the model gives 5.4, one of 22 levels 9.7 for 6.0.  The last
+// terms are fits: 48x40x24 takes 171 us per solve with 180 boxes of class 1, 206
+// with 504 and 200 with 252 of class 0, 24x20x16 170 with 16 boxes, 200 with one.
 static double res_cost(const ResShape& h, int words, int on) {
   const int waves = h.nthr / kWave, kl = h.kl, over = kl - (h.cls == 0 ? 32 : 16);
   const double slow = over <= 0 ? 1.0 : over <= 2 ? 1.25 : over <= 4 ? 1.4 : over <= 6 ? 1.65 : 2.0;
   const double sweep = std::max(0.034 * ((on * waves + 3) / 4), 0.055) * kl + 0.3 + 0.05 * waves * on;
-  const double cross = h.nb > 1 ? 1.5 + 0.35 * on * words / 1024 : 0.0;
-  return slow * (on == 1 ? sweep + cross : std::max(sweep, 0.6 * sweep + cross));
+  const double cross = 1.5 + 0.35 * on * words / 1024;
+  if (h.nb == 1) return sweep + 0.6;
+  if (on == 1) return slow * (sweep + cross) - (h.cls == 1 ? 0.35 : 0.0);
+  return slow * std::max(sweep, 0.6 * sweep + cross);
 }
 
 static int up(int a, int b) { return (a + b - 1) / b; }
@@ -1045,7 +1053,7 @@ static void launch_res(const ResGrid& r, const ResArgs& a) {
   RES(12)
   RES(16)
   // (every two levels where registers spill: 300x300x90, boxes of 18 levels,
-  // takes 680 us per solve, in the kernel for 20 levels 760)
+  // took 680 us per solve, in the kernel for 20 levels 760)
   if constexpr (CLS == 1) RES(18)
   RES(20)
   if constexpr (CLS == 1) RES(22)
