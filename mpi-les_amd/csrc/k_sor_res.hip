@@ -59,7 +59,7 @@ constexpr int res_lds_rhs(int cls, int bk) {
   const int room = (163840 / kResClass[cls].per - 512 - 4 * bk * kResClass[cls].plane) / (4 * kResNT);
   return cls == 0 ? 0 : room < bk ? room : bk;
 }
-constexpr long long kEnterTicks = 100000;  // 1 ms of the 100 MHz wall clock
+constexpr long long kEnterTicks = 1000000;  // 10 ms of the 100 MHz wall clock
 constexpr int kSpinMax = 1 << 22;  // polls of one word before the solve is given up (seconds)
 
 __device__ __forceinline__ int rcix(const SplitGrid& s, int t, int j, int k) {

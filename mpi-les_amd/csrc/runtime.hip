@@ -9,6 +9,7 @@
 
 #include <algorithm>
 #include <array>
+#include <atomic>
 #include <condition_variable>
 #include <map>
 #include <mutex>
@@ -741,7 +742,12 @@ float omega_default = 1.0f;
 // enqueued work holding one is ordered, per device, after the work holding
 // the one before, when that is on another stream: an event recorded there
 // now.  The lock is held while the work is enqueued.
+// While such domains exist the steps of all domains take their turn so: blocks
+// waiting for their fellows hold compute units that another domain's kernel
+// would need to end and make room (mixed sizes on streams of their own ran 10
+// times slower).
 std::mutex g_res_mu;
+std::atomic<int> g_res_domains{0};
 struct ResLast {
   hipStream_t stream = nullptr;
   hipEvent_t ev = nullptr;
@@ -798,6 +804,7 @@ void domain_free(les_domain* D) {
   dev_release(D->d.ctrl);
   dev_release(D->d.partials);
   dev_release(D->d.dc64);
+  if (D->d.res_mem) g_res_domains--;
   dev_release(D->d.res_mem);
   res_forget(D->d.stream);
   stream_destroy(D->d.stream);
@@ -939,6 +946,7 @@ int domain_alloc(int im, int jm, int km, les_domain** out) {
     if (e == hipSuccess) e = hipMemsetAsync(D->d.res_mem, 0, nb, D->d.stream);
     if (e != hipSuccess) return bail(std::string("SOR workspace allocation: ") + hipGetErrorString(e));
     D->bytes += (long long)nb;
+    g_res_domains++;
   }
   // SOR partial slots for any k chunk of the fused iteration (down to one
   // level per block) and for the colour sweeps
@@ -1593,7 +1601,7 @@ int les_press(int km, int jm, int im, float* rhs, const float* u, const float* d
   D->d.pjuge = pjuge_default;
   D->d.omega = omega_default;
   if (flush_metrics(D)) return 1;
-  ResOrder order(press_resident(D->d), D->d.stream);
+  ResOrder order(g_res_domains > 0, D->d.stream);
   HIP_TRY(order.err);
   return run_stage(D, 6, n, nmax);
 }
@@ -1935,7 +1943,7 @@ int les_domain_destroy(les_domain* D) {
 int les_domain_stage(les_domain* D, int stage, int n, int nmax) {
   if (!live_has(D)) return fail("null, unknown or destroyed domain");
   if (flush_metrics(D)) return 1;
-  ResOrder order(stage == 6 && press_resident(D->d), D->d.stream);
+  ResOrder order(g_res_domains > 0, D->d.stream);
   HIP_TRY(order.err);
   return run_stage(D, stage, n, nmax);
 }
@@ -1984,7 +1992,7 @@ static int step_graph(les_domain* D, int n, int nmax) {
 int les_domain_step(les_domain* D, int n, int nmax) {
   if (!live_has(D)) return fail("null, unknown or destroyed domain");
   if (flush_metrics(D)) return 1;  // may allow or rule out the one-launch SOR
-  ResOrder order(press_resident(D->d), D->d.stream);
+  ResOrder order(g_res_domains > 0, D->d.stream);
   HIP_TRY(order.err);
   if (D->use_graph && n != 1 && !D->d.timer) return step_graph(D, n, nmax);
   return run_step(D, n, nmax);
@@ -2430,6 +2438,8 @@ int batch_enqueue(les_batch* B, const int* ns, const int* nmaxs, bool capturing)
   HIP_TRY(hipEventRecord(B->fork, B->stream));
   std::vector<char> split(nd, 0);
   int res_prev = -1;
+  bool any_res = false;
+  for (const les_domain* D : B->doms) any_res = any_res || press_resident(D->d);
   for (size_t q = 0; q < nd; q++) {
     les_domain* D = B->doms[q];
     D->rhs_lazy = D->d.press_mode == 0;  // a batched press also leaves the split rhs equal to rhs
@@ -2442,8 +2452,8 @@ int batch_enqueue(les_batch* B, const int* ns, const int* nmaxs, bool capturing)
       continue;
     }
     HIP_TRY(hipStreamWaitEvent(D->d.stream, B->fork, 0));
-    // those running the one-launch SOR on their own step one after the other
-    if ((!B->full[q] || B->res[q]) && press_resident(D->d)) {
+    // beside a one-launch SOR, those on their own step one after the other
+    if (any_res) {
       if (res_prev >= 0) HIP_TRY(hipStreamWaitEvent(D->d.stream, B->head_done[res_prev], 0));
       res_prev = (int)q;
     }
@@ -2550,10 +2560,7 @@ int les_batch_step(les_batch* B, const int* ns, const int* nmaxs) {
     if (flush_metrics(D)) return 1;  // synchronous: not under capture
     D->rhs_lazy = D->d.press_mode == 0;
   }
-  bool res = false;  // a domain runs the one-launch SOR, on its own stream or beside others
-  for (size_t q = 0; q < B->doms.size(); q++)
-    res = res || ((!B->full[q] || B->res[q]) && press_resident(B->doms[q]->d));
-  ResOrder order(res, B->stream);
+  ResOrder order(g_res_domains > 0, B->stream);
   HIP_TRY(order.err);
   bool replay = B->use_graph != 0;
   for (size_t q = 0; q < B->doms.size(); q++) replay = replay && ns[q] != 1;
