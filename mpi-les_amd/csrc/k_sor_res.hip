@@ -903,11 +903,17 @@ bool res_shape(const Grid& g, const SplitGrid& s, int units, ResShape* out) {
 // modelled time of the slowest domain.  From its fewest boxes each domain takes
 // more while it is the slowest and they fit.  Returns the time, negative when
 // no kernel holds them all.
-static double res_batch_cut(const DevDomain* const* all, const std::vector<int>& ds, int units, ResShape* shapes) {
-  struct Cut {
-    ResShape h;
-    double cost;
-  };
+struct Cut {
+  ResShape h;
+  double cost;
+};
+// A domain's cuts by class and levels / 4, made when first asked for.
+struct Cuts {
+  std::vector<Cut> v[2][16];
+  bool have[2][16] = {};
+};
+static double res_batch_cut(const DevDomain* const* all, const std::vector<int>& ds, int units, ResShape* shapes,
+                            std::vector<Cuts>& memo) {
   double best = -1.0;
   for (int cls = 0; cls < 2; cls++) {
     const int cap = kResClass[cls].per * units;
@@ -917,6 +923,13 @@ static double res_batch_cut(const DevDomain* const* all, const std::vector<int>&
       bool ok = true;
       for (size_t q = 0; q < ds.size() && ok; q++) {
         const DevDomain& d = *all[ds[q]];
+        Cuts& mm = memo[ds[q]];
+        if (mm.have[cls][bk / 4]) {
+          cuts[q] = mm.v[cls][bk / 4];
+          ok = !cuts[q].empty();
+          if (ok) total += cuts[q][0].h.nb + 1;
+          continue;
+        }
         std::vector<Cut> v;
         res_cuts(d.g, d.sg, cls, cap - 1, bk - 4, bk, [&](const ResShape& h, int wds) {
           v.push_back({h, res_cost(h, wds, cls == 1 ? 2 : 1)});
@@ -930,6 +943,8 @@ static double res_batch_cut(const DevDomain* const* all, const std::vector<int>&
           else
             w.push_back(c);
         }
+        mm.v[cls][bk / 4] = cuts[q];
+        mm.have[cls][bk / 4] = true;
         ok = !cuts[q].empty();
         if (ok) total += cuts[q][0].h.nb + 1;
       }
@@ -968,12 +983,13 @@ double res_batch_plan(const DevDomain* const* ds, int n, int units, ResShape* sh
   // as few launches as hold them, or more while that is faster
   double best = -1.0;
   std::vector<ResShape> sh(n);
+  std::vector<Cuts> memo(n);
   for (int ng = 1; ng <= n; ng++) {
     std::vector<std::vector<int>> in(ng);  // dealt out there and back
     for (int r = 0; r < n; r++) in[(r / ng) & 1 ? ng - 1 - r % ng : r % ng].push_back(by[r]);
     double sum = 0.0;
     for (const auto& v : in) {
-      const double c = res_batch_cut(ds, v, units, sh.data());
+      const double c = res_batch_cut(ds, v, units, sh.data(), memo);
       if (c < 0.0) {
         sum = -1.0;
         break;
