@@ -2017,6 +2017,8 @@ int les_domain_autotune(les_domain* D, int reps, int* rows, int* tile_rows, int*
   auto it = g_tuned.find(key);
   if (it == g_tuned.end() || reps > 0) {
     TuneResult t;
+    ResOrder order(g_res_domains > 0, D->d.stream);  // its trials end before the next step is enqueued
+    HIP_TRY(order.err);
     if (tune_sor(D, reps > 0 ? reps : 10, &t)) return 1;
     if (tune_stencils(D, reps > 0 ? reps : 10, &t)) return 1;
     it = g_tuned.insert_or_assign(key, t).first;
@@ -2055,6 +2057,8 @@ int les_domain_time_sor(les_domain* D, int iters, double* us_per_iter) {
   if (!D || !us_per_iter) return fail("null argument");
   if (iters < 1) return fail("les_domain_time_sor: iters < 1");
   if (!D->d.sor_fused) return fail("les_domain_time_sor: the fused SOR iteration is off");
+  ResOrder order(g_res_domains > 0, D->d.stream);
+  HIP_TRY(order.err);
   HIP_TRY(hipStreamSynchronize(D->d.stream));
   Ctrl saved;
   HIP_TRY(copy_sync(&saved, D->d.ctrl, sizeof(Ctrl), hipMemcpyDeviceToHost, D->d.stream));
