@@ -311,6 +311,11 @@ int les_selftest_reciprocal(unsigned lo_bits, unsigned hi_bits, unsigned long lo
 long long les_domain_bytes_needed(int im, int jm, int km);
 int les_domain_press_stats(les_domain* d, int* iters, double* sor_hist, int hist_len, double* rhsav,
                            double* pav, int* nonfinite);
+/* Pressure solves of the domain that were to run in one launch, found part of
+ * the device held by other work for 10 ms, and completed in a slower form (with
+ * the same results).  After one the next steps use the kernels that need no
+ * whole device.  Synchronises.  No reference counterpart. */
+int les_domain_solve_fallbacks(les_domain* d, int* count);
 /* Bytes of device memory the domain holds. */
 long long les_domain_bytes(const les_domain* d);
 

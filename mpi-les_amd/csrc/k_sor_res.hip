@@ -60,6 +60,8 @@ constexpr int res_lds_rhs(int cls, int bk) {
   return cls == 0 ? 0 : room < bk ? room : bk;
 }
 constexpr long long kEnterTicks = 1000000;  // 10 ms of the 100 MHz wall clock
+constexpr int kEnterShift = 6;  // ... and 0.16 after as many solves in a row by tickets
+constexpr int kTickets = 128;   // pieces a sweep is handed out in, at most
 constexpr int kSpinMax = 1 << 22;  // polls of one word before the solve is given up (seconds)
 
 __device__ __forceinline__ int rcix(const SplitGrid& s, int t, int j, int k) {
@@ -201,25 +203,32 @@ __device__ __forceinline__ int res_verdict(ConstArgs a, int np, int l, unsigned 
 
 // 1: every block of the launch is resident; 2: they are not, and the launch
 // runs by tickets.  Thread 0 of each block; the last block to arrive decides
-// 1, a block that waited kEnterTicks (or force_ticket) decides 2, whichever
-// comes first.
+// 1, a block that waited kEnterTicks decides 2, whichever comes first.  Where
+// the launches before went by tickets the wait is shorter, for work that holds
+// the device mostly goes on holding it: steps enqueued ahead would pay it each.
 __device__ __forceinline__ void res_arrive(Ctrl* ctrl, int nb) {
   const int n = __hip_atomic_fetch_add(&ctrl->res_arrived, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   if (n == nb - 1) {
     int want = 0;
-    __hip_atomic_compare_exchange_strong(&ctrl->res_state, &want, 1, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
-                                         __HIP_MEMORY_SCOPE_AGENT);
+    if (__hip_atomic_compare_exchange_strong(&ctrl->res_state, &want, 1, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                             __HIP_MEMORY_SCOPE_AGENT))
+      ast(&ctrl->res_short, 0);
   }
 }
-__device__ __forceinline__ int res_enter(Ctrl* ctrl) {
-  const long long t0 = wall_clock64();
+__device__ __forceinline__ int res_enter(Ctrl* ctrl, int* note) {
+  const long long t0 = wall_clock64(), patience = kEnterTicks >> min(ald(&ctrl->res_short), kEnterShift);
   for (;;) {
     const int st = ald(&ctrl->res_state);
     if (st != 0) return st;
-    if (wall_clock64() - t0 > kEnterTicks) {
+    if (wall_clock64() - t0 > patience) {
       int want = 0;
-      __hip_atomic_compare_exchange_strong(&ctrl->res_state, &want, 2, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
-                                           __HIP_MEMORY_SCOPE_AGENT);
+      if (__hip_atomic_compare_exchange_strong(&ctrl->res_state, &want, 2, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                               __HIP_MEMORY_SCOPE_AGENT)) {
+        ast(&ctrl->res_short, ald(&ctrl->res_short) + 1);
+        // the solves of a domain follow each other: one writer at a time
+        const int n = __hip_atomic_load(note, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        __hip_atomic_store(note, n + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+      }
       return ald(&ctrl->res_state);
     }
     __builtin_amdgcn_s_sleep(1);
@@ -241,8 +250,15 @@ __device__ __forceinline__ void res_ticket(ConstArgs a0, float* lds_f, double av
   const int im = g.im, jm = g.jm, km = g.km, nt = s.nt;
   if (a->nred > 0 && blockIdx.x == 0 && tid == 0) ctrl->rhsav = av;
   const int npr = nt * jm;                          // pairs per level
-  const int chunks = (npr + nthr - 1) / nthr;      // tickets per level
-  const int per = chunks * km;                      // tickets per sweep
+  const int chunks = (npr + nthr - 1) / nthr;      // pieces of a level, a pair to each thread
+  const int items = chunks * km;
+  // pieces per ticket: kTickets tickets per sweep.  Each costs its place in two
+  // counters and the fences that carry a sweep from one block to another: a
+  // step of 300x300x90 took 170 ms with a ticket per piece (7920 per sweep), 34
+  // with 990, 14.1 with 256, 12.7 with 128 and 17.5 with 64; 96x96x64 17.7, 9.7, 4.2,
+  // 4.3 and 4.3.
+  const int span = (items + kTickets - 1) / kTickets;
+  const int per = (items + span - 1) / span;        // tickets per sweep
   for (;;) {
     __syncthreads();
     if (tid == 0)
@@ -270,9 +286,10 @@ __device__ __forceinline__ void res_ticket(ConstArgs a0, float* lds_f, double av
     if (sh[1] != 0) return;
     const int l = (sweep + 1) / 2, col = sweep & 1;  // col 1 = red
     const int src = (l - 1) & 1, dst = l & 1;
-    const int x = (it % chunks) * nthr + tid, k = 1 + it / chunks;
     double acc = 0.0;
-    if (x < npr) {
+    for (int m = it * span; m < min(items, (it + 1) * span); m++) {
+      const int x = (m % chunks) * nthr + tid, k = 1 + m / chunks;
+      if (x >= npr) continue;
       const int t = x % nt, j = 1 + x / nt;
       const int q = rcix(s, t, j, k);
       if (sweep == 0) {
@@ -311,7 +328,7 @@ __device__ __forceinline__ void res_ticket(ConstArgs a0, float* lds_f, double av
                                                           a->sb.rhs[col][q]) -
                                        own);
           a->sb.p[dst][col][q] = own + rel;
-          acc = (double)rel * (double)rel;
+          acc += (double)rel * (double)rel;
         }
       }
     }
@@ -364,10 +381,10 @@ __device__ __forceinline__ void res_block(ConstArgs a0, const int bid) {
   const int nb = a0->nb;
   // sor_done set on entry (a finished defect correction): nothing to solve
   const bool skip = a0->ctrl->sor_done != 0;  // (no block passes res_enter, to change it, before all have read it)
-  if (tid == 0 && !skip && !a0->force_ticket) res_arrive(a0->ctrl, nb + 1);
+  if (tid == 0 && !skip && !a0->force_ticket) res_arrive(a0->ctrl, nb + 1 + a0->missing);
   const double av = a0->nred > 0 ? res_mean(again(a0), tid, nthr, wsum) : 0.0;  // while the others arrive
   if (tid == 0) {
-    sh[0] = skip ? 0 : a0->force_ticket ? 2 : res_enter(a0->ctrl);
+    sh[0] = skip ? 0 : a0->force_ticket ? 2 : res_enter(a0->ctrl, a0->note);
     sh[1] = 0;
     av_s = av;  // read where the rhs is
   }
@@ -1010,11 +1027,8 @@ double res_batch_plan(const DevDomain* const* ds, int n, int units, ResShape* sh
 // 8-byte words of the workspace: inboxes of both colours, the partial sums
 // of four iterations (two words each) and their verdicts, and the partial sums of the ticket
 // sweeps.
-static long res_tickets(const Grid& g, const SplitGrid& s) {
-  return (long)((s.nt * (long)g.jm + 63) / 64) * g.km;  // blocks of at least 64 threads
-}
-long res_words(const Grid& g, const SplitGrid& s, const ResShape& h) {
-  return 2L * h.nb * h.iw + 8L * h.nb * (h.nthr / kWave) + 8 + 4 * res_tickets(g, s);
+long res_words(const ResShape& h) {
+  return 2L * h.nb * h.iw + 8L * h.nb * (h.nthr / kWave) + 8 + 4 * kTickets;
 }
 
 ResArgs res_args(const DevDomain& d, const ResShape& h, unsigned long long* mem, const SplitBufs& sb, int nmaxp,
@@ -1036,6 +1050,8 @@ ResArgs res_args(const DevDomain& d, const ResShape& h, unsigned long long* mem,
   a.nmaxp = nmaxp;
   a.zero = zero;
   a.force_ticket = d.res_on == 2;
+  a.missing = d.res_on == 3;
+  a.note = d.res_note;
   a.ntx = h.ntx;
   a.nty = h.nty;
   a.ntz = h.ntz;

@@ -77,6 +77,7 @@ struct Ctrl {
   // the solve (the words of earlier ones are told by it), blocks that have
   // entered, 1 all resident / 2 by tickets, and the ticket counters
   int res_epoch, res_arrived, res_state, tk_next, tk_phase, tk_done;
+  int res_short;           // solves in a row that went by tickets, their blocks not all running in time
   double rhsav;            // volume-weighted mean of rhs
   double pav;              // volume-weighted mean of p
   double sor_first;        // sum of reltmp^2 of the current iteration's first colour

@@ -64,6 +64,8 @@ struct ResArgs {
   double* tparts;              // partial sums of the ticket sweeps
   float c2, c3, omega, pjuge;  // uniform cn2l = cn2s, cn3l = cn3s
   int nmaxp, zero, force_ticket;  // zero: start from p = 0 instead of pent
+  int missing;                 // blocks waited for that the launch does not have (0; 1 in tests: the wait times out)
+  int* note;                   // host memory: solves whose blocks were not all running in time
   int ntx, nty, ntz, tp, tj, kl, nb, iw, nq;
 };
 
@@ -120,17 +122,19 @@ struct DevDomain {
   // masks of that form; nullptr for other masks (the fields are read)
   const float* mask_src;
   // the one-launch SOR: 1 used where the grid fits and is uniform in i and j
-  // (2: always by tickets), its boxes, workspace and uniform coefficients
+  // (2: always by tickets; 3: waits for a block too many, then by tickets),
+  // its boxes, workspace, host counter and uniform coefficients
   int res_on, res_uniform;
   ResShape res;
   unsigned long long* res_mem;
+  int* res_note;
   float res_c2, res_c3;
 };
 
 // The one-launch SOR (k_sor_res.hip): the boxes of a domain on ncu compute
 // units (false: it does not fit) and the 8-byte words of its workspace.
 bool res_shape(const Grid& g, const SplitGrid& s, int ncu, ResShape* out);
-long res_words(const Grid& g, const SplitGrid& s, const ResShape& h);
+long res_words(const ResShape& h);
 inline bool use_res(const DevDomain& d) { return d.res_on && d.res_uniform && d.cn1_separable; }
 // Whether a press runs it, for its solve or for the inner ones of mode 1.
 inline bool press_resident(const DevDomain& d) {

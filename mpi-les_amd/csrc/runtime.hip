@@ -117,6 +117,47 @@ void dev_release(void* p) {
   g_pool_live.erase(it);
 }
 
+// Host words that kernels count in (DevDomain::res_note), a cache line each,
+// from pinned pages.  les_release_all gives the pages back when no domain
+// holds a word.
+constexpr size_t kNotePage = 4096, kNoteLine = 64;
+std::mutex g_note_mu;
+std::vector<int*> g_note_pages, g_note_free;
+
+int* note_take() {
+  std::lock_guard<std::recursive_mutex> ck(g_capture_mu);
+  std::lock_guard<std::mutex> lk(g_note_mu);
+  if (g_note_free.empty()) {
+    char* p = nullptr;
+    if (hipHostMalloc((void**)&p, kNotePage, hipHostMallocDefault) != hipSuccess) {
+      (void)hipGetLastError();
+      return nullptr;
+    }
+    g_note_pages.push_back((int*)p);
+    for (size_t o = 0; o < kNotePage; o += kNoteLine) g_note_free.push_back((int*)(p + o));
+  }
+  int* n = g_note_free.back();
+  g_note_free.pop_back();
+  __atomic_store_n(n, 0, __ATOMIC_RELAXED);
+  return n;
+}
+
+// No kernel that writes the word may still run.
+void note_return(int* n) {
+  if (!n) return;
+  std::lock_guard<std::mutex> lk(g_note_mu);
+  g_note_free.push_back(n);
+}
+
+void notes_trim() {
+  std::lock_guard<std::recursive_mutex> ck(g_capture_mu);
+  std::lock_guard<std::mutex> lk(g_note_mu);
+  if (g_note_free.size() != g_note_pages.size() * (kNotePage / kNoteLine)) return;
+  for (int* p : g_note_pages) hipHostFree(p);
+  g_note_pages.clear();
+  g_note_free.clear();
+}
+
 hipError_t stream_create(hipStream_t* s) {
   std::lock_guard<std::recursive_mutex> ck(g_capture_mu);
   return hipStreamCreateWithFlags(s, hipStreamNonBlocking);
@@ -435,6 +476,9 @@ struct les_domain {
   // since it was last written); a download gathers it first
   bool rhs_lazy = false;
   double st_us_best = 0.0, st_us_default = 0.0;  // the stencil tuner's timings for this shape
+  // The one-launch SOR: DevDomain::res_on as asked for, the solves by tickets
+  // seen so far, and the steps left before it is tried again after one.
+  int res_want = 0, res_seen = 0, res_rest = 0, res_pause = 0, res_good = 0;
 };
 
 namespace {
@@ -781,6 +825,30 @@ void res_forget(hipStream_t s) {
     if (kv.second.stream == s) kv.second.stream = nullptr;
 }
 
+// A one-launch solve whose blocks found no room (work of another process, or
+// work of this one that is not ordered by ResOrder) has waited and then gone by
+// tickets, which takes many times as long.  The steps after it run the
+// launch-per-iterations kernels, which share the device: kPauseMin of them, and
+// twice as many each time another solve finds no room soon after.
+constexpr int kPauseMin = 32, kPauseMax = 4096;
+void res_review(les_domain* D) {
+  if (!D->d.res_note || D->res_want == 2) return;
+  const int n = __atomic_load_n(D->d.res_note, __ATOMIC_RELAXED);
+  if (n != D->res_seen) {
+    D->res_seen = n;
+    if (D->d.res_on) {  // else a solve enqueued before the pause
+      D->res_pause = D->res_pause == 0 ? kPauseMin : std::min(2 * D->res_pause, kPauseMax);
+      D->d.res_on = 0;
+    }
+    D->res_rest = D->res_pause;
+    D->res_good = 0;
+  } else if (!D->d.res_on) {
+    if (--D->res_rest <= 0) D->d.res_on = D->res_want;
+  } else if (D->res_pause > 0 && ++D->res_good > D->res_pause) {
+    D->res_pause = 0;
+  }
+}
+
 void timer_free(les_domain* D) {
   Timer* T = (Timer*)D->d.timer;
   if (!T) return;
@@ -806,6 +874,7 @@ void domain_free(les_domain* D) {
   dev_release(D->d.dc64);
   if (D->d.res_mem) g_res_domains--;
   dev_release(D->d.res_mem);
+  note_return(D->d.res_note);
   res_forget(D->d.stream);
   stream_destroy(D->d.stream);
   delete D;
@@ -941,12 +1010,15 @@ int domain_alloc(int im, int jm, int km, les_domain** out) {
     if (getenv(v)) D->d.res_on = 0;
   if (D->d.res_on && !res_shape(D->d.g, D->d.sg, D->d.ncu > 0 ? D->d.ncu : 256, &D->d.res)) D->d.res_on = 0;
   if (D->d.res_on) {
-    const size_t nb = (size_t)res_words(D->d.g, D->d.sg, D->d.res) * 8;
+    const size_t nb = (size_t)res_words(D->d.res) * 8;
     e = dev_alloc(&D->d.res_mem, nb);
     if (e == hipSuccess) e = hipMemsetAsync(D->d.res_mem, 0, nb, D->d.stream);
     if (e != hipSuccess) return bail(std::string("SOR workspace allocation: ") + hipGetErrorString(e));
     D->bytes += (long long)nb;
     g_res_domains++;
+    D->d.res_note = note_take();
+    if (!D->d.res_note) D->d.res_on = 0;
+    D->res_want = D->d.res_on;
   }
   // SOR partial slots for any k chunk of the fused iteration (down to one
   // level per block) and for the colour sweeps
@@ -1601,6 +1673,7 @@ int les_press(int km, int jm, int im, float* rhs, const float* u, const float* d
   D->d.pjuge = pjuge_default;
   D->d.omega = omega_default;
   if (flush_metrics(D)) return 1;
+  res_review(D);
   ResOrder order(g_res_domains > 0, D->d.stream);
   HIP_TRY(order.err);
   return run_stage(D, 6, n, nmax);
@@ -1714,6 +1787,7 @@ int les_release_all(void) {
   g_domains.clear();
   g_inflows.clear();
   rings_trim();
+  notes_trim();
   pool_trim();
   return 0;
 }
@@ -1926,7 +2000,7 @@ long long les_domain_bytes_needed(int im, int jm, int km) {
     Grid g{im, jm, km, (int)sj, 0};
     SplitGrid s{(int)nt, (int)cp, 0};
     ResShape h;
-    if (res_shape(g, s, ncu, &h)) b += 8LL * res_words(g, s, h);  // the one-launch SOR
+    if (res_shape(g, s, ncu, &h)) b += 8LL * res_words(h);  // the one-launch SOR
   }
   b += ((long long)im * jm + km) * 4;  // the masks' column values and level thresholds
   return b + (1LL << 20);  // metrics, partial sums, control block (bounded by 1 MiB here)
@@ -1943,6 +2017,7 @@ int les_domain_destroy(les_domain* D) {
 int les_domain_stage(les_domain* D, int stage, int n, int nmax) {
   if (!live_has(D)) return fail("null, unknown or destroyed domain");
   if (flush_metrics(D)) return 1;
+  if (stage == 6) res_review(D);
   ResOrder order(g_res_domains > 0, D->d.stream);
   HIP_TRY(order.err);
   return run_stage(D, stage, n, nmax);
@@ -1992,6 +2067,7 @@ static int step_graph(les_domain* D, int n, int nmax) {
 int les_domain_step(les_domain* D, int n, int nmax) {
   if (!live_has(D)) return fail("null, unknown or destroyed domain");
   if (flush_metrics(D)) return 1;  // may allow or rule out the one-launch SOR
+  res_review(D);
   ResOrder order(g_res_domains > 0, D->d.stream);
   HIP_TRY(order.err);
   if (D->use_graph && n != 1 && !D->d.timer) return step_graph(D, n, nmax);
@@ -2124,6 +2200,14 @@ int les_domain_press_stats(les_domain* D, int* iters, double* sor_hist, int hist
                            double* pav, int* nonfinite) {
   if (!live_has(D)) return fail("null, unknown or destroyed domain");
   return read_stats(D, iters, sor_hist, hist_len, rhsav, pav, nonfinite);
+}
+
+int les_domain_solve_fallbacks(les_domain* D, int* count) {
+  if (!live_has(D)) return fail("null, unknown or destroyed domain");
+  if (!count) return fail("null argument");
+  HIP_TRY(hipStreamSynchronize(D->d.stream));
+  *count = D->d.res_note ? __atomic_load_n(D->d.res_note, __ATOMIC_RELAXED) : 0;
+  return 0;
 }
 
 long long les_domain_bytes(const les_domain* D) { return live_has(D) ? D->bytes : 0; }
@@ -2270,7 +2354,7 @@ int batch_res_prepare(les_batch* B) {
   std::vector<int> b0s;
   const size_t ntab = (nd * sizeof(ResArgs) + 255) / 256 * 256, nb0 = (nd * sizeof(int) + 255) / 256 * 256;
   size_t words = 0;
-  for (int r = 0; r < nd; r++) words += (size_t)(res_words(ds[r]->g, ds[r]->sg, sh[r]) + 31) / 32 * 32;
+  for (int r = 0; r < nd; r++) words += (size_t)(res_words(sh[r]) + 31) / 32 * 32;
   HIP_TRY(dev_alloc(&B->res_mem, ntab + nb0 + 8 * words));
   char* const base = (char*)B->res_mem;
   unsigned long long* mem = (unsigned long long*)(base + ntab + nb0);
@@ -2285,7 +2369,7 @@ int batch_res_prepare(les_batch* B) {
       SplitBufs sb = d.sb;
       sb.cn1[0] = sb.cn1[1] = nullptr;  // separable cn1
       tab.push_back(res_args(d, sh[r], mem, sb, d.nmaxp, d.pjuge, d.omega, false));
-      mem += (size_t)(res_words(d.g, d.sg, sh[r]) + 31) / 32 * 32;
+      mem += (size_t)(res_words(sh[r]) + 31) / 32 * 32;
       b0s.push_back(L.blocks);
       L.blocks += sh[r].nb + 1;
       L.nd++;
@@ -2552,6 +2636,16 @@ int les_batch_step(les_batch* B, const int* ns, const int* nmaxs) {
   if (!live_has(B) || !ns || !nmaxs) return fail("les_batch_step: null argument, or unknown or destroyed batch");
   for (les_domain* D : B->doms)  // a domain must outlive the batches holding it
     if (!live_has(D)) return fail("les_batch_step: a domain of the batch was destroyed");
+  int rest = 0;  // the pauses of the domains are one pause of the batch
+  for (les_domain* D : B->doms) {
+    res_review(D);
+    if (!D->d.res_on && D->res_want) rest = std::max(rest, D->res_rest);
+  }
+  for (les_domain* D : B->doms)
+    if (rest > 0 && D->res_want && D->res_want != 2) {
+      D->d.res_on = 0;
+      D->res_rest = rest;
+    }
   if (!batch_key_same(B)) {
     if (B->gexec) {
       HIP_TRY(hipStreamSynchronize(B->stream));

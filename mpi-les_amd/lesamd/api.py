@@ -97,6 +97,7 @@ def lib():
     L.les_domain_bytes_needed.argtypes = [ci, ci, ci]
     L.les_domain_bytes_needed.restype = ctypes.c_longlong
     L.les_domain_press_stats.argtypes = [vp, vp, vp, ci, vp, vp, vp]
+    L.les_domain_solve_fallbacks.argtypes = [vp, vp]
     L.les_domain_bytes.argtypes = [vp]
     L.les_domain_bytes.restype = ctypes.c_longlong
     L.les_domain_set_timing.argtypes = [vp, ci]
@@ -300,6 +301,13 @@ class Domain:
         """True when the last pressure solve met a non-finite residual (the
         state has diverged).  Waits for the domain's stream."""
         return self.press_stats()["nonfinite"] != 0
+
+    def solve_fallbacks(self) -> int:
+        """Pressure solves that found part of the GPU held by other work and
+        completed in the slower form.  Waits for the domain's stream."""
+        n = ctypes.c_int()
+        _check(lib().les_domain_solve_fallbacks(self._h, ctypes.byref(n)))
+        return n.value
 
     def autotune(self, reps: int = 0) -> dict:
         """Pick the SOR launch shape and the stencil kernels' k levels per
