@@ -3,13 +3,13 @@
 // conversion, and the C ABI declared in include/les_amd.h.
 #include <math.h>
 #include <cmath>
+#include <pthread.h>
 #include <stdio.h>
 #include <stdlib.h>
 #include <string.h>
 
 #include <algorithm>
 #include <array>
-#include <atomic>
 #include <condition_variable>
 #include <map>
 #include <mutex>
@@ -21,6 +21,7 @@
 
 #include "../../include/les_amd.h"
 #include "les_kernels.h"
+#include "turns.h"
 
 using namespace les;
 
@@ -55,6 +56,9 @@ std::mutex g_pool_mu;
 std::multimap<std::pair<int, size_t>, void*> g_pool_kept;  // (device, bytes) -> block
 std::map<void*, std::pair<int, size_t>> g_pool_live;
 std::recursive_mutex g_capture_mu;
+// Held while a stream is captured, and while an event is recorded on a stream
+// of another domain or batch (which must not be under capture).
+std::mutex g_record_mu;
 
 void pool_trim() {
   std::lock_guard<std::recursive_mutex> ck(g_capture_mu);
@@ -780,53 +784,50 @@ int nmaxp_default = 50;
 float pjuge_default = 1.0e-4f;
 float omega_default = 1.0f;
 
-// The solves of k_sor_res need every compute unit they were cut for at once:
-// two of them running side by side would each hold units the other waits
-// for, until both fall back to their slow form.  So in this process the
-// enqueued work holding one is ordered, per device, after the work holding
-// the one before, when that is on another stream: an event recorded there
-// now.  The lock is held while the work is enqueued.
-// While such domains exist the steps of all domains take their turn so: blocks
-// waiting for their fellows hold compute units that another domain's kernel
-// would need to end and make room (mixed sizes on streams of their own ran 10
-// times slower).
-std::mutex g_res_mu;
-std::atomic<int> g_res_domains{0};
-struct ResLast {
-  hipStream_t stream = nullptr;
+// The turns of steps and solves on each device (turns.h).  Whole-device work is
+// enqueued with the lock held alone, other work beside each other; g_turn_mu
+// guards the state itself.  Uploads, downloads, statistics and the set-up of a
+// domain take no turn: they end by themselves soon.
+pthread_rwlock_t g_turn_lock = PTHREAD_RWLOCK_WRITER_NONRECURSIVE_INITIALIZER_NP;
+std::mutex g_turn_mu;
+struct DevTurns {
+  Turns<hipStream_t> turns;
   hipEvent_t ev = nullptr;
 };
-std::map<int, ResLast> g_res_last;
+std::map<int, DevTurns> g_turns;
 
-struct ResOrder {
-  std::unique_lock<std::mutex> lk;
+// Held while work is enqueued on s.  whole: it holds a one-launch solve.
+struct Turn {
   hipError_t err = hipSuccess;
-  ResOrder(bool on, hipStream_t s) {
-    if (!on) return;
-    lk = std::unique_lock<std::mutex>(g_res_mu);
+  Turn(bool whole, hipStream_t s) {
+    if (whole)
+      pthread_rwlock_wrlock(&g_turn_lock);
+    else
+      pthread_rwlock_rdlock(&g_turn_lock);
     int dev = 0;
     if ((err = hipGetDevice(&dev)) != hipSuccess) return;
-    ResLast& l = g_res_last[dev];
-    if (l.stream && l.stream != s) {
-      std::lock_guard<std::recursive_mutex> ck(g_capture_mu);  // neither stream is being captured
-      if (!l.ev) err = hipEventCreateWithFlags(&l.ev, hipEventDisableTiming);
-      if (err == hipSuccess) err = hipEventRecord(l.ev, l.stream);
-      if (err == hipSuccess) err = hipStreamWaitEvent(s, l.ev, 0);
-      if (err != hipSuccess) return;
-    }
-    l.stream = s;
+    std::lock_guard<std::mutex> lk(g_turn_mu);
+    DevTurns& d = g_turns[dev];
+    d.turns.take(s, whole, [&](hipStream_t t, hipStream_t to) {
+      std::lock_guard<std::mutex> ck(g_record_mu);  // t is not being captured
+      if (!d.ev) err = hipEventCreateWithFlags(&d.ev, hipEventDisableTiming);
+      if (err == hipSuccess) err = hipEventRecord(d.ev, t);
+      if (err == hipSuccess) err = hipStreamWaitEvent(to, d.ev, 0);
+      return (int)(err != hipSuccess);
+    });
   }
+  ~Turn() { pthread_rwlock_unlock(&g_turn_lock); }
+  Turn(const Turn&) = delete;
 };
 
 // The stream goes away (its work is complete).
-void res_forget(hipStream_t s) {
-  std::lock_guard<std::mutex> lk(g_res_mu);
-  for (auto& kv : g_res_last)
-    if (kv.second.stream == s) kv.second.stream = nullptr;
+void turn_forget(hipStream_t s) {
+  std::lock_guard<std::mutex> lk(g_turn_mu);
+  for (auto& kv : g_turns) kv.second.turns.forget(s);
 }
 
 // A one-launch solve whose blocks found no room (work of another process, or
-// work of this one that is not ordered by ResOrder) has waited and then gone by
+// work of this one that takes no turn) has waited and then gone by
 // tickets, which takes many times as long.  The steps after it run the
 // launch-per-iterations kernels, which share the device: kPauseMin of them, and
 // twice as many each time another solve finds no room soon after.
@@ -872,10 +873,9 @@ void domain_free(les_domain* D) {
   dev_release(D->d.ctrl);
   dev_release(D->d.partials);
   dev_release(D->d.dc64);
-  if (D->d.res_mem) g_res_domains--;
   dev_release(D->d.res_mem);
   note_return(D->d.res_note);
-  res_forget(D->d.stream);
+  turn_forget(D->d.stream);
   stream_destroy(D->d.stream);
   delete D;
 }
@@ -1015,7 +1015,6 @@ int domain_alloc(int im, int jm, int km, les_domain** out) {
     if (e == hipSuccess) e = hipMemsetAsync(D->d.res_mem, 0, nb, D->d.stream);
     if (e != hipSuccess) return bail(std::string("SOR workspace allocation: ") + hipGetErrorString(e));
     D->bytes += (long long)nb;
-    g_res_domains++;
     D->d.res_note = note_take();
     if (!D->d.res_note) D->d.res_on = 0;
     D->res_want = D->d.res_on;
@@ -1221,14 +1220,19 @@ int time_sor_trial(les_domain* D, const Ctrl& base, int rows, int ty, int tw, in
   Ctrl c = base;
   c.sor_done = 0;
   c.nonfinite = 0;
-  hipError_t e = hipMemcpyAsync(D->d.ctrl, &c, sizeof(Ctrl), hipMemcpyHostToDevice, D->d.stream);
-  if (e == hipSuccess) {
-    launch_sor_trial(D->d, rows, ty, tw, kc, 2);  // warm-up
-    e = hipEventRecord(e0, D->d.stream);
-  }
-  if (e == hipSuccess) {
-    launch_sor_trial(D->d, rows, ty, tw, kc, reps);
-    e = hipEventRecord(e1, D->d.stream);
+  hipError_t e;
+  {
+    Turn turn(false, D->d.stream);
+    e = turn.err;
+    if (e == hipSuccess) e = hipMemcpyAsync(D->d.ctrl, &c, sizeof(Ctrl), hipMemcpyHostToDevice, D->d.stream);
+    if (e == hipSuccess) {
+      launch_sor_trial(D->d, rows, ty, tw, kc, 2);  // warm-up
+      e = hipEventRecord(e0, D->d.stream);
+    }
+    if (e == hipSuccess) {
+      launch_sor_trial(D->d, rows, ty, tw, kc, reps);
+      e = hipEventRecord(e1, D->d.stream);
+    }
   }
   if (e == hipSuccess) e = hipEventSynchronize(e1);
   float ms = 0.0f;
@@ -1375,16 +1379,21 @@ int tune_stencils(les_domain* D, int reps, TuneResult* r) {
     d.velfg_kchunk = vkc;
     d.sm_kchunk = skc;
     d.visc_kchunk = ckc;
-    hipError_t te = copy_all(true);
-    for (int q = -1; q < reps && te == hipSuccess; q++) {
-      if (q == 0) te = hipEventRecord(e0, d.stream);
-      if (which == 0)
-        launch_velfg_feedbf(d, D->vn, D->alpha, D->dt, D->beta);
-      else
-        launch_les_adam(d);
-      if (te == hipSuccess) te = hipGetLastError();
+    hipError_t te;
+    {
+      Turn turn(false, d.stream);
+      te = turn.err;
+      if (te == hipSuccess) te = copy_all(true);
+      for (int q = -1; q < reps && te == hipSuccess; q++) {
+        if (q == 0) te = hipEventRecord(e0, d.stream);
+        if (which == 0)
+          launch_velfg_feedbf(d, D->vn, D->alpha, D->dt, D->beta);
+        else
+          launch_les_adam(d);
+        if (te == hipSuccess) te = hipGetLastError();
+      }
+      if (te == hipSuccess) te = hipEventRecord(e1, d.stream);
     }
-    if (te == hipSuccess) te = hipEventRecord(e1, d.stream);
     if (te == hipSuccess) te = hipEventSynchronize(e1);
     float ms = 0.0f;
     if (te == hipSuccess) te = hipEventElapsedTime(&ms, e0, e1);
@@ -1674,8 +1683,8 @@ int les_press(int km, int jm, int im, float* rhs, const float* u, const float* d
   D->d.omega = omega_default;
   if (flush_metrics(D)) return 1;
   res_review(D);
-  ResOrder order(g_res_domains > 0, D->d.stream);
-  HIP_TRY(order.err);
+  Turn turn(press_resident(D->d), D->d.stream);
+  HIP_TRY(turn.err);
   return run_stage(D, 6, n, nmax);
 }
 
@@ -2018,18 +2027,17 @@ int les_domain_stage(les_domain* D, int stage, int n, int nmax) {
   if (!live_has(D)) return fail("null, unknown or destroyed domain");
   if (flush_metrics(D)) return 1;
   if (stage == 6) res_review(D);
-  ResOrder order(g_res_domains > 0, D->d.stream);
-  HIP_TRY(order.err);
+  Turn turn(stage == 6 && press_resident(D->d), D->d.stream);
+  HIP_TRY(turn.err);
   return run_stage(D, stage, n, nmax);
 }
 
-// One step from a graph captured on the domain's stream.  Every launch
+// The graph of a step, captured on the domain's stream.  Every launch
 // argument of a step n > 1 is fixed by the domain state (pointers, sizes,
 // physical constants, SOR controls), so one capture serves every such step;
 // a change of that state triggers a new capture.  Step 1 differs (initial
 // copy in bondv1) and runs eagerly.
-static int step_graph(les_domain* D, int n, int nmax) {
-  if (flush_metrics(D)) return 1;
+static int step_capture(les_domain* D, int n, int nmax) {
   const float sc[5] = {D->ro, D->vn, D->alpha, D->beta, D->dt};
   if (D->gexec && (memcmp(&D->gkey, &D->d, sizeof(DevDomain)) != 0 || memcmp(D->gscal, sc, sizeof(sc)) != 0)) {
     HIP_TRY(hipStreamSynchronize(D->d.stream));  // the previous replay may still be running
@@ -2040,6 +2048,7 @@ static int step_graph(les_domain* D, int n, int nmax) {
     // allocations cannot be captured: make the stage scratch exist first
     if (!D->d.fuse_velfg && ensure_cov(D)) return 1;
     std::lock_guard<std::recursive_mutex> ck(g_capture_mu);
+    std::lock_guard<std::mutex> rk(g_record_mu);
     HIP_TRY(hipStreamBeginCapture(D->d.stream, hipStreamCaptureModeThreadLocal));
     int rc = 0;
     rc = run_step(D, n, nmax);
@@ -2059,8 +2068,6 @@ static int step_graph(les_domain* D, int n, int nmax) {
     memcpy(&D->gkey, &D->d, sizeof(DevDomain));
     memcpy(D->gscal, sc, sizeof(sc));
   }
-  HIP_TRY(hipGraphLaunch(D->gexec, D->d.stream));
-  D->rhs_lazy = D->d.press_mode == 0;
   return 0;
 }
 
@@ -2068,10 +2075,14 @@ int les_domain_step(les_domain* D, int n, int nmax) {
   if (!live_has(D)) return fail("null, unknown or destroyed domain");
   if (flush_metrics(D)) return 1;  // may allow or rule out the one-launch SOR
   res_review(D);
-  ResOrder order(g_res_domains > 0, D->d.stream);
-  HIP_TRY(order.err);
-  if (D->use_graph && n != 1 && !D->d.timer) return step_graph(D, n, nmax);
-  return run_step(D, n, nmax);
+  const bool replay = D->use_graph && n != 1 && !D->d.timer;
+  if (replay && step_capture(D, n, nmax)) return 1;
+  Turn turn(press_resident(D->d), D->d.stream);
+  HIP_TRY(turn.err);
+  if (!replay) return run_step(D, n, nmax);
+  HIP_TRY(hipGraphLaunch(D->gexec, D->d.stream));
+  D->rhs_lazy = D->d.press_mode == 0;
+  return 0;
 }
 
 int les_domain_aveflow(les_domain* D, int n, int n1, int nmax) {
@@ -2093,8 +2104,6 @@ int les_domain_autotune(les_domain* D, int reps, int* rows, int* tile_rows, int*
   auto it = g_tuned.find(key);
   if (it == g_tuned.end() || reps > 0) {
     TuneResult t;
-    ResOrder order(g_res_domains > 0, D->d.stream);  // its trials end before the next step is enqueued
-    HIP_TRY(order.err);
     if (tune_sor(D, reps > 0 ? reps : 10, &t)) return 1;
     if (tune_stencils(D, reps > 0 ? reps : 10, &t)) return 1;
     it = g_tuned.insert_or_assign(key, t).first;
@@ -2133,8 +2142,6 @@ int les_domain_time_sor(les_domain* D, int iters, double* us_per_iter) {
   if (!D || !us_per_iter) return fail("null argument");
   if (iters < 1) return fail("les_domain_time_sor: iters < 1");
   if (!D->d.sor_fused) return fail("les_domain_time_sor: the fused SOR iteration is off");
-  ResOrder order(g_res_domains > 0, D->d.stream);
-  HIP_TRY(order.err);
   HIP_TRY(hipStreamSynchronize(D->d.stream));
   Ctrl saved;
   HIP_TRY(copy_sync(&saved, D->d.ctrl, sizeof(Ctrl), hipMemcpyDeviceToHost, D->d.stream));
@@ -2298,7 +2305,7 @@ void batch_free(les_batch* B) {
   for (hipEvent_t e : B->tail_done) hipEventDestroy(e);
   if (B->fork) hipEventDestroy(B->fork);
   if (B->sor_done) hipEventDestroy(B->sor_done);
-  res_forget(B->stream);
+  turn_forget(B->stream);
   stream_destroy(B->stream);
   delete B;
 }
@@ -2658,15 +2665,16 @@ int les_batch_step(les_batch* B, const int* ns, const int* nmaxs) {
     if (flush_metrics(D)) return 1;  // synchronous: not under capture
     D->rhs_lazy = D->d.press_mode == 0;
   }
-  ResOrder order(g_res_domains > 0, B->stream);
-  HIP_TRY(order.err);
+  bool whole = false;  // some domain solves in one launch
+  for (size_t q = 0; q < B->doms.size(); q++)
+    whole = whole || B->res[q] || (!B->full[q] && press_resident(B->doms[q]->d));
   bool replay = B->use_graph != 0;
   for (size_t q = 0; q < B->doms.size(); q++) replay = replay && ns[q] != 1;
-  if (!replay) return batch_enqueue(B, ns, nmaxs, false);
-  if (!B->gexec) {
+  if (replay && !B->gexec) {
     for (les_domain* D : B->doms)
       if (!D->d.fuse_velfg && ensure_cov(D)) return 1;  // allocations cannot be captured
     std::lock_guard<std::recursive_mutex> ck(g_capture_mu);
+    std::lock_guard<std::mutex> rk(g_record_mu);
     HIP_TRY(hipStreamBeginCapture(B->stream, hipStreamCaptureModeThreadLocal));
     const int rc = batch_enqueue(B, ns, nmaxs, true);
     hipGraph_t gr = nullptr;
@@ -2683,6 +2691,9 @@ int les_batch_step(les_batch* B, const int* ns, const int* nmaxs) {
       return fail(std::string("hipGraphInstantiate: ") + hipGetErrorString(ei));
     }
   }
+  Turn turn(whole, B->stream);
+  HIP_TRY(turn.err);
+  if (!replay) return batch_enqueue(B, ns, nmaxs, false);
   // a graph runs on the batch stream only: order it after the domains'
   // streams and their later work after it
   for (size_t q = 0; q < B->doms.size(); q++) {
