@@ -16,7 +16,6 @@ batched-step path (les_domain_step, les_batch_step), unchanged.
 """
 from __future__ import annotations
 
-import os
 import dataclasses
 import math
 import time
@@ -210,7 +209,6 @@ class Server:
     def __init__(self, budget_bytes: int, burst: int = 4, max_active: int = 64, domain_factory=None,
                  bytes_of=None, clock=time.perf_counter, batch_factory=None, workers: int = 1):
         self.budget = int(budget_bytes)
-        self._mixed = False  # the run steps large domains on their own streams beside a batch
         self.burst = int(burst)
         self.max_active = int(max_active)
         self.clock = clock
@@ -220,16 +218,7 @@ class Server:
             from . import api
 
             def factory(req):
-                # one-launch pressure solves need the whole GPU at once: beside large
-                # domains on streams of their own they ran 3 times slower than without
-                old = os.environ.get("LES_SOR_RESIDENT")
-                if self._mixed and old is None:
-                    os.environ["LES_SOR_RESIDENT"] = "0"
-                try:
-                    d = api.Domain(setup_gen.build(req.workload, dense=False))
-                finally:
-                    if self._mixed and old is None:
-                        os.environ.pop("LES_SOR_RESIDENT", None)
+                d = api.Domain(setup_gen.build(req.workload, dense=False))
                 d.set_graph(True)
                 d.autotune()  # SOR launch shape and stencil k levels for this grid shape (timed once per shape)
                 return d
@@ -270,7 +259,6 @@ class Server:
         GPU by themselves, replay their own step graphs on their own streams
         alongside.  Requests join at step boundaries once their domain is
         ready, and leave when their last step has completed."""
-        self._mixed = max_batch_cells is not None and any(r.cells > max_batch_cells for r in requests)
         lc = _Lifecycle(self, requests, self.max_active, self.clock())
         batched: list[_Active] = []
         alone: list[_Active] = []
