@@ -1010,12 +1010,19 @@ int domain_alloc(int im, int jm, int km, les_domain** out) {
     if (getenv(v)) D->d.res_on = 0;
   if (D->d.res_on && !res_shape(D->d.g, D->d.sg, D->d.ncu > 0 ? D->d.ncu : 256, &D->d.res)) D->d.res_on = 0;
   if (D->d.res_on) {
+    // a device without room for its workspace runs the other kernels
     const size_t nb = (size_t)res_words(D->d.res) * 8;
     e = dev_alloc(&D->d.res_mem, nb);
-    if (e == hipSuccess) e = hipMemsetAsync(D->d.res_mem, 0, nb, D->d.stream);
-    if (e != hipSuccess) return bail(std::string("SOR workspace allocation: ") + hipGetErrorString(e));
-    D->bytes += (long long)nb;
-    D->d.res_note = note_take();
+    if (e == hipErrorOutOfMemory)
+      (void)hipGetLastError();
+    else if (e == hipSuccess)
+      e = hipMemsetAsync(D->d.res_mem, 0, nb, D->d.stream);
+    if (e != hipSuccess && e != hipErrorOutOfMemory)
+      return bail(std::string("SOR workspace allocation: ") + hipGetErrorString(e));
+    if (e == hipSuccess) {
+      D->bytes += (long long)nb;
+      D->d.res_note = note_take();
+    }
     if (!D->d.res_note) D->d.res_on = 0;
     D->res_want = D->d.res_on;
   }
@@ -2362,7 +2369,12 @@ int batch_res_prepare(les_batch* B) {
   const size_t ntab = (nd * sizeof(ResArgs) + 255) / 256 * 256, nb0 = (nd * sizeof(int) + 255) / 256 * 256;
   size_t words = 0;
   for (int r = 0; r < nd; r++) words += (size_t)(res_words(sh[r]) + 31) / 32 * 32;
-  HIP_TRY(dev_alloc(&B->res_mem, ntab + nb0 + 8 * words));
+  const hipError_t ea = dev_alloc(&B->res_mem, ntab + nb0 + 8 * words);
+  if (ea == hipErrorOutOfMemory) {  // no room for the workspaces: one launch per iteration
+    (void)hipGetLastError();
+    return 0;
+  }
+  HIP_TRY(ea);
   char* const base = (char*)B->res_mem;
   unsigned long long* mem = (unsigned long long*)(base + ntab + nb0);
   for (int q = 0; q < ng; q++) {
