@@ -50,6 +50,13 @@ METRIC = "steps/s + Mcell-updates/s at 300x300x90 FP32, %HBM peak; served p50/p9
 # iteration, pressure-mean removal 12).
 STEP_BYTES_FIXED = 40 + 60 + 64 + 64 + 48 + 28 + 12
 SOR_BYTES_PER_ITER = 12
+# The one-launch SOR keeps its iterates in registers: it reads the start iterate
+# and the rhs once and writes the rhs (its mean removed) and the last iterate.
+# Its rate is that of the vector ALU: 17 operations per cell and iteration, of
+# which 256 CUs issue 64 lanes each per cycle at 2.4 GHz.
+SOR_ONE_LAUNCH_BYTES = 16
+SOR_OPS_PER_ITER = 17
+VALU_PEAK_TOPS = 256 * 64 * 2.4e9 / 1e12
 SOR_RUN = 200  # back-to-back SOR launches timed for the dominant kernel's duration
 # per launch of each kernel class, bytes per interior cell (sor: per iteration)
 CLASS_BYTES = {
@@ -58,6 +65,27 @@ CLASS_BYTES = {
 }
 STATE_FIELDS = ("u", "v", "w", "p", "f", "g", "h", "usum", "vsum", "wsum", "fold", "gold", "hold", "rhs",
                 "sm", "uspd", "vspd") + tuple(f"diu{q}" for q in range(1, 10))
+
+
+def sor_roofline(cells: int, iters_per_launch: float, launch_s: float, resident: bool) -> dict:
+    """Rate of a SOR launch against what bounds it: the HBM bytes of its
+    iterations, or (resident: all iterations of a press in one launch, the
+    iterates in registers) the operations of the vector ALU, with the bytes
+    the launch itself cannot do without beside them."""
+    if resident:
+        achieved = cells * iters_per_launch * SOR_OPS_PER_ITER / launch_s / 1e12
+        return {"bound": "valu", "achieved": round(achieved, 2), "peak": round(VALU_PEAK_TOPS, 1), "unit": "Top/s",
+                "frac": round(achieved / VALU_PEAK_TOPS, 4),
+                "alg_bytes_per_launch": int(SOR_ONE_LAUNCH_BYTES * cells)}
+    nbytes = SOR_BYTES_PER_ITER * cells * iters_per_launch
+    achieved = nbytes / launch_s / 1e9
+    return {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
+            "frac": round(achieved / HBM_PEAK_GBS, 4), "alg_bytes_per_launch": int(nbytes)}
+
+
+def step_bytes(cells: int, iters: int, resident: bool) -> int:
+    """Bytes a step cannot do without, by the kernels it runs."""
+    return cells * (STEP_BYTES_FIXED + (SOR_ONE_LAUNCH_BYTES if resident else SOR_BYTES_PER_ITER * iters))
 
 
 def _time_steps(be, n0, nsteps, budget_s):
@@ -208,7 +236,7 @@ def serve_measurement(nreq: int, nsteps: int, sizes=None, rate: float | None = N
         "arrivals": f"Poisson, {rate:g} requests/s" if rate else "all at t=0",
         "offered_mcell_updates_per_s": round(offered, 1) if offered else None,
         "mode": f"continuous batching of the domains of at most {SERVE_BATCH_CELLS} cells (each stage one launch "
-                "for all of them, SOR one launch per iteration), larger domains on their own streams",
+                "for all of them, the SOR too where the domains qualify), larger domains on their own streams",
         "mcell_updates_per_s": round(bat["mcell_updates_per_s"], 1),
         "p50_s": round(bat["p50_s"], 4), "p99_s": round(bat["p99_s"], 4), "failed": bat["failed"],
         "speedup_vs_sequential": round(bat["mcell_updates_per_s"] / seq["mcell_updates_per_s"], 3),
@@ -555,7 +583,6 @@ def main(argv=None):
     dom_cls = max((c for c in kt if kt[c][1] > 0), key=lambda c: kt[c][0])
     dom_ms, dom_n = kt[dom_cls]
     avg_s = dom_ms / 1e3 / dom_n
-    alg_bytes = CLASS_BYTES.get(dom_cls, 0) * w.cells
     fused = os.environ.get("LES_SOR_FUSED", "1") != "0"
     # one launch per step and no class "sor1": all iterations in one launch
     resident = kt.get("sor1", (0.0, 0))[1] == 0 and kt["sor"][1] == K and L > 1
@@ -566,7 +593,6 @@ def main(argv=None):
     ipl = 0.5 if not fused else (2 if sor_rows == 4 else 1)
     if dom_cls == "sor" and resident:
         ipl = sum(iters_run) / dom_n
-        alg_bytes = SOR_BYTES_PER_ITER * w.cells * ipl
     elif dom_cls == "sor":
         # Class "sor" holds the SOR launches after the one holding iteration
         # 1 (class "sor1"), or all colour sweeps (LES_SOR_FUSED=0).
@@ -575,7 +601,6 @@ def main(argv=None):
         # time is divided among the launches that carried them.
         first = {0.5: 0, 1: 1, 2: 2}[ipl]
         iters = sum(max(0, it - first) for it in iters_run)
-        alg_bytes = SOR_BYTES_PER_ITER * w.cells * ipl
         avg_s = dom_ms / 1e3 / max(1, round(iters / ipl))
     in_step_us = avg_s * 1e6
     timing_method = "one HIP event pair per launch in K eager steps"
@@ -587,8 +612,12 @@ def main(argv=None):
         avg_s = dom.time_sor(SOR_RUN) * ipl / 1e6
         timing_method = (f"one HIP event pair around {SOR_RUN} back-to-back iterations "
                          f"({int(SOR_RUN / ipl)} launches) on the domain's stream")
-    achieved = alg_bytes / avg_s / 1e9
-    step_bytes = w.cells * (STEP_BYTES_FIXED + SOR_BYTES_PER_ITER * L)
+    if dom_cls == "sor":
+        rate = sor_roofline(w.cells, ipl, avg_s, resident)
+    else:
+        nbytes = CLASS_BYTES.get(dom_cls, 0) * w.cells
+        rate = {"bound": "hbm", "achieved": round(nbytes / avg_s / 1e9, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
+                "frac": round(nbytes / avg_s / 1e9 / HBM_PEAK_GBS, 4), "alg_bytes_per_launch": nbytes}
     per_kernel = {c: {"ms_per_step": round(v[0] / nprof, 4), "launches_per_step": v[1] / nprof,
                       "us_per_launch": round(1e3 * v[0] / v[1], 2)} for c, v in kt_all.items() if v[1]}
 
@@ -609,16 +638,11 @@ def main(argv=None):
                    "nmaxp": w.nmaxp, "pjuge": w.pjuge, "seed": w.seed},
         "mcell_updates_per_s": round(sps * w.cells / 1e6, 2),
         "sor_iters_last_step": L,
-        "hbm_frac_step": round(step_bytes * sps / 1e9 / HBM_PEAK_GBS, 4),
+        "hbm_frac_step": round(step_bytes(w.cells, L, resident) * sps / 1e9 / HBM_PEAK_GBS, 4),
         "roofline": {
             "kernel": dom_cls,
-            "bound": "hbm",
-            "achieved": round(achieved, 1),
-            "peak": HBM_PEAK_GBS,
-            "unit": "GB/s",
-            "frac": round(achieved / HBM_PEAK_GBS, 4),
+            **rate,
             "traffic": profiled_traffic(dom_cls, w.name, sor_rows, resident),
-            "alg_bytes_per_launch": int(alg_bytes),
             "sor_iterations_per_launch": ipl if dom_cls == "sor" else None,
             "avg_launch_us": round(avg_s * 1e6, 3),
             "timing": timing_method,
