@@ -210,17 +210,17 @@ __device__ __forceinline__ void res_arrive(Ctrl* ctrl, int nb) {
   const int n = __hip_atomic_fetch_add(&ctrl->res_arrived, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   if (n == nb - 1) {
     int want = 0;
-    if (__hip_atomic_compare_exchange_strong(&ctrl->res_state, &want, 1, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
-                                             __HIP_MEMORY_SCOPE_AGENT))
-      ast(&ctrl->res_short, 0);
+    __hip_atomic_compare_exchange_strong(&ctrl->res_state, &want, 1, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                         __HIP_MEMORY_SCOPE_AGENT);
   }
 }
 __device__ __forceinline__ int res_enter(Ctrl* ctrl, int* note) {
-  const long long t0 = wall_clock64(), patience = kEnterTicks >> min(ald(&ctrl->res_short), kEnterShift);
+  const long long t0 = wall_clock64();
   for (;;) {
     const int st = ald(&ctrl->res_state);
     if (st != 0) return st;
-    if (wall_clock64() - t0 > patience) {
+    const long long t = wall_clock64() - t0;
+    if (t > (kEnterTicks >> kEnterShift) && t > (kEnterTicks >> min(ald(&ctrl->res_short), kEnterShift))) {
       int want = 0;
       if (__hip_atomic_compare_exchange_strong(&ctrl->res_state, &want, 2, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
                                                __HIP_MEMORY_SCOPE_AGENT)) {
@@ -396,6 +396,7 @@ __device__ __forceinline__ void res_block(ConstArgs a0, const int bid) {
     return;
   }
   if (bid == nb) {
+    if (tid == 0) ast(&a0->ctrl->res_short, 0);
     res_monitor(again(a0), nb, (unsigned)a0->ctrl->res_epoch * 8192u, tid, nthr, wsum);
     return;
   }
