@@ -7,7 +7,6 @@ import os
 import numpy as np
 import pytest
 
-import test_gpu_autotune as autotune
 import test_gpu_batch as batch
 from lesamd import api, setup_gen
 
@@ -30,8 +29,23 @@ def test_batch_staggered_joins(per_iteration, monkeypatch):
 
 @pytest.mark.parametrize("case", [dict(im=90, jm=40, km=24, seed=31), dict(im=61, jm=27, km=18, seed=32)],
                          ids=lambda c: f"{c['im']}x{c['jm']}x{c['km']}")
-def test_autotune_keeps_state_and_results(case, per_iteration):
-    autotune.test_autotune_keeps_state_and_results(case)
+def test_a_tuned_domain_steps_like_an_untuned_one(case, per_iteration):
+    s = setup_gen.build(setup_gen.small_workload(**case))
+    print(f"\n[tuned, per iteration] {case}", flush=True)
+    a, b = api.Domain(s), api.Domain(s)
+    r = a.autotune(reps=4)
+    assert r["rows"] in ((1, 2, 4) if case["jm"] % 2 == 0 else (1,)), r
+    assert 0.0 < r["us_per_iter"] <= r["us_per_iter_default"], r
+    for n in range(1, 5):
+        a.step(n, 4)
+        b.step(n, 4)
+    for f in batch.FIELDS:
+        assert np.array_equal(a.download(f), b.download(f)), f
+    x, y = a.press_stats(), b.press_stats()
+    assert x["iters"] == y["iters"]
+    np.testing.assert_allclose(x["sor"], y["sor"], rtol=1e-12, atol=0)
+    a.close()
+    b.close()
 
 
 @pytest.mark.parametrize("graph", [True, False], ids=["graph", "eager"])
