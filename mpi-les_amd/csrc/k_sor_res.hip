@@ -1051,7 +1051,7 @@ ResArgs res_args(const DevDomain& d, const ResShape& h, unsigned long long* mem,
   a.nmaxp = nmaxp;
   a.zero = zero;
   a.force_ticket = d.res_on == 2;
-  a.missing = d.res_on == 3;
+  a.missing = d.res_on == 3 || (d.res_on == 4 && __atomic_load_n(d.res_note, __ATOMIC_RELAXED) == 0);
   a.note = d.res_note;
   a.ntx = h.ntx;
   a.nty = h.nty;

@@ -122,7 +122,8 @@ struct DevDomain {
   // masks of that form; nullptr for other masks (the fields are read)
   const float* mask_src;
   // the one-launch SOR: 1 used where the grid fits and is uniform in i and j
-  // (2: always by tickets; 3: waits for a block too many, then by tickets),
+  // (2: always by tickets; 3: waits for a block too many, then by tickets; 4:
+  // so until the first solve of that kind is noted),
   // its boxes, workspace, host counter and uniform coefficients
   int res_on, res_uniform;
   ResShape res;

@@ -453,6 +453,13 @@ void les::timer_end(const DevDomain& d, int c) {
   T->chain = true;
 }
 
+// After a one-launch solve that found no room (res_review): 0 in use, 1 paused,
+// 2 tried in one step and paused until that is known to have gone well.
+struct ResPause {
+  int phase = 0, rest = 0;    // steps left in the phase
+  int length = 0, good = 0;   // of the last pause (0: none lately); steps in use since
+};
+
 struct les_domain {
   DevDomain d{};
   int n3 = 0;                       // floats per 3-D field
@@ -481,8 +488,9 @@ struct les_domain {
   bool rhs_lazy = false;
   double st_us_best = 0.0, st_us_default = 0.0;  // the stencil tuner's timings for this shape
   // The one-launch SOR: DevDomain::res_on as asked for, the solves by tickets
-  // seen so far, and the steps left before it is tried again after one.
-  int res_want = 0, res_seen = 0, res_rest = 0, res_pause = 0, res_good = 0;
+  // seen so far, and where the domain stands after one (res_review).
+  int res_want = 0, res_seen = 0;
+  ResPause res_pause;
 };
 
 namespace {
@@ -827,26 +835,40 @@ void turn_forget(hipStream_t s) {
 }
 
 // A one-launch solve whose blocks found no room (work of another process, or
-// work of this one that takes no turn) has waited and then gone by
-// tickets, which takes many times as long.  The steps after it run the
+// work of this one that takes no turn) has waited and then gone by tickets,
+// which takes many times as long.  The steps after it run the
 // launch-per-iterations kernels, which share the device: kPauseMin of them, and
-// twice as many each time another solve finds no room soon after.
-constexpr int kPauseMin = 32, kPauseMax = 4096;
+// twice as many each time it is tried again in vain.  Tried again it is in one
+// step; the next kProbe do not follow its example yet, for steps may be
+// enqueued long before they run.  A step in vain costs as much as 20 (300x300x90)
+// or more, the other kernels 0.2 ms a step.  Two processes stepping 300x300x90 each on one GPU
+// take 2.83 ms a step with the other kernels alone.
+constexpr int kPauseMin = 256, kPauseMax = 16384, kProbe = 32;
 void res_review(les_domain* D) {
   if (!D->d.res_note || D->res_want == 2) return;
+  ResPause& P = D->res_pause;
   const int n = __atomic_load_n(D->d.res_note, __ATOMIC_RELAXED);
   if (n != D->res_seen) {
     D->res_seen = n;
-    if (D->d.res_on) {  // else a solve enqueued before the pause
-      D->res_pause = D->res_pause == 0 ? kPauseMin : std::min(2 * D->res_pause, kPauseMax);
-      D->d.res_on = 0;
+    if (P.phase != 1)  // else a solve enqueued before the pause
+      P.length = P.length == 0 ? kPauseMin : std::min(2 * P.length, kPauseMax);
+    P.phase = 1;
+    P.rest = P.length;
+    D->d.res_on = 0;
+  } else if (P.phase == 1) {
+    if (--P.rest <= 0) {
+      P.phase = 2;
+      P.rest = kProbe;
+      D->d.res_on = D->res_want;
     }
-    D->res_rest = D->res_pause;
-    D->res_good = 0;
-  } else if (!D->d.res_on) {
-    if (--D->res_rest <= 0) D->d.res_on = D->res_want;
-  } else if (D->res_pause > 0 && ++D->res_good > D->res_pause) {
-    D->res_pause = 0;
+  } else if (P.phase == 2) {
+    D->d.res_on = 0;
+    if (--P.rest <= 0) {
+      P.phase = P.good = 0;
+      D->d.res_on = D->res_want;
+    }
+  } else if (P.length > 0 && ++P.good > P.length) {
+    P.length = 0;
   }
 }
 
@@ -2676,15 +2698,16 @@ int les_batch_step(les_batch* B, const int* ns, const int* nmaxs) {
   if (!live_has(B) || !ns || !nmaxs) return fail("les_batch_step: null argument, or unknown or destroyed batch");
   for (les_domain* D : B->doms)  // a domain must outlive the batches holding it
     if (!live_has(D)) return fail("les_batch_step: a domain of the batch was destroyed");
-  int rest = 0;  // the pauses of the domains are one pause of the batch
+  // a pause of one domain is one of the batch, the longest of theirs
+  const les_domain* paused = nullptr;
   for (les_domain* D : B->doms) {
     res_review(D);
-    if (!D->d.res_on && D->res_want) rest = std::max(rest, D->res_rest);
+    if (D->res_pause.phase != 0 && (!paused || D->res_pause.rest > paused->res_pause.rest)) paused = D;
   }
   for (les_domain* D : B->doms)
-    if (rest > 0 && D->res_want && D->res_want != 2) {
-      D->d.res_on = 0;
-      D->res_rest = rest;
+    if (paused && D->d.res_note && D->res_want != 2) {
+      D->res_pause = paused->res_pause;
+      D->d.res_on = paused->d.res_on ? D->res_want : 0;
     }
   if (!batch_key_same(B)) {
     if (B->gexec) {

@@ -1,8 +1,9 @@
 """The decision of the one-launch SOR (k_sor_res) to solve by tickets when its
 blocks are not all running in time, forced with LES_SOR_RESIDENT=3 (each block
-waits for one block more than the launch has), and what the domain does after
-it: the next steps run the launch-per-iterations kernels, twice as many after
-each further solve of that kind.  Fields bit for bit as with
+waits for one block more than the launch has; 4: until one such solve is noted),
+and what the domain does after it: the next steps run the launch-per-iterations
+kernels, twice as many after each further solve of that kind, then one step
+tries the one launch again.  Fields bit for bit as with
 LES_SOR_RESIDENT=0, the stop-test sums to the rounding of their order."""
 import dataclasses
 import os
@@ -14,7 +15,8 @@ from lesamd import api, setup_gen
 
 pytestmark = pytest.mark.gpu
 FIELDS = ("p", "u", "v", "w", "rhs")
-PAUSE = 32  # steps without the one-launch solve after the first that went by tickets
+PAUSE = 256  # steps without the one-launch solve after the first that went by tickets
+PROBE = 32   # ... and after the step that tries it again
 
 
 def _domain(s, mode):
@@ -52,6 +54,32 @@ def test_a_solve_without_room_pauses_the_one_launch_form(dims, graph):
     assert [n + 1 for n in range(nmax) if n == 0 or seen[n] != seen[n - 1]] == [1, PAUSE + 2, 3 * PAUSE + 3], seen
     assert seen[0] == 1 and seen[-1] == 3
     assert ref.solve_fallbacks() == 0
+    ref.close()
+    dom.close()
+
+
+@pytest.mark.parametrize("graph", [False, True], ids=["eager", "graph"])
+def test_room_again_brings_the_one_launch_form_back(graph):
+    """The first solve finds no room, later ones do.  The launches per step
+    tell the form: one SOR launch in the one-launch form."""
+    s = setup_gen.build(dataclasses.replace(setup_gen.small_workload(40, 28, 14, seed=9), nmaxp=6), dense=False)
+    print(f"\n[sor fallback] room again, graph {graph}", flush=True)
+    ref, dom = _domain(s, 0), _domain(s, 4)
+    dom.set_graph(graph)
+    nmax = PAUSE + PROBE + 12
+    for n in range(1, nmax + 1):
+        ref.step(n, nmax)
+        at = (1, 2, PAUSE + 1, PAUSE + 2, PAUSE + 3, PAUSE + PROBE + 1, PAUSE + PROBE + 2, nmax)
+        if n in at:
+            dom.set_timing(True)
+        dom.step(n, nmax)
+        if n in at:
+            kt = dom.timing()
+            one = (kt["sor"][1], kt["sor1"][1]) == (1, 0)
+            dom.set_timing(False)
+            assert one == (n in (1, PAUSE + 2, PAUSE + PROBE + 2, nmax)), n
+            _same(ref, dom, n)
+        assert dom.solve_fallbacks() == 1
     ref.close()
     dom.close()
 
