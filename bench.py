@@ -244,7 +244,8 @@ def serve_measurement(nreq: int, nsteps: int, sizes=None, rate: float | None = N
         "sequential_p50_s": round(seq["p50_s"], 4), "sequential_p99_s": round(seq["p99_s"], 4),
         "sequential_failed": seq["failed"],
         "fp64_oracle_error": "the same as one-at-a-time runs: served fields are bit-identical to the domain "
-                             "stepped alone (tests/test_gpu_batch.py, tests/test_gpu_configs.py)",
+                             "stepped alone (tests/test_gpu_batch.py, tests/test_gpu_batch_routes.py, "
+                             "tests/test_gpu_configs.py)",
     }
     if con is not None:
         out.update({"streams_mcell_updates_per_s": round(con["mcell_updates_per_s"], 1),

@@ -322,14 +322,16 @@ long long les_domain_bytes(const les_domain* d);
 /* ------------------------------------------------------------ batches
  * Several domains advanced together, one step of each per les_batch_step.
  * Domains with a batchable whole step (fused reference SOR, separable cn1,
- * even jm, velfg+feedbf and les+adam fused) run every stage as one launch
+ * velfg+feedbf and les+adam fused, and even jm unless the domain solves in one
+ * launch) run every stage as one launch
  * for all of them: each block runs its own domain's stage on that domain's
  * grid, and the SOR runs as one launch (domains whose solve fits the device's
  * registers, side by side), or iterations 2..nmaxp as one launch per iteration
  * with one k chunk for the batch (LES_BATCH_SOR_KCHUNK and
- * LES_BATCH_SOR_TILE_ROWS override it).  A step in which such a domain has
- * n == 1 runs its stages on its own stream and only the SOR iterations
- * batched.  Other domains step whole on their own streams, joined by
+ * LES_BATCH_SOR_TILE_ROWS override it).  In a step in which such a domain has
+ * n == 1 they run their stages on their own streams, those that solve in one
+ * launch their SOR too, the others only the SOR iterations batched.  Other
+ * domains step whole on their own streams, joined by
  * events.  With the graph on (default), steps where every n > 1 replay one
  * graph (recaptured when a domain's state changes).  Fields and SOR
  * iteration counts are those of stepping each domain alone, bit for bit;

@@ -2,8 +2,8 @@
 // iterates and the right-hand side stay in the registers of the whole GPU
 // from the first iteration to the last.
 //
-// A domain is cut into nb boxes of pairs x rows x levels, one per block and
-// at most one block per compute unit.  A thread owns one (pair, row) column
+// A domain is cut into nb boxes of pairs x rows x levels, one per block, with
+// one block or two per compute unit (kResClass).  A thread owns one (pair, row) column
 // of its box -- red and black cell of each level, their rhs, in registers --
 // so the k neighbours are its own values; the in-plane neighbours come from
 // one LDS copy of the colour last updated, with a ring of halo cells around
@@ -15,23 +15,27 @@
 //
 // What bounds it: the exchange on small domains (one word crosses between two
 // compute units in 1 us, and a solve of 50 iterations waits for 100 of them
-// in a row), the vector ALU on large ones (19 instructions per cell, four
-// waves per SIMD; at 300x300x90 about 4 us of each 7.8 us sweep).  The
+// in a row); on large ones the vector ALU (37 lane-instructions per cell and
+// iteration, 377 of the 656 us of a solve at 300x300x90) and the words (2.7 GB
+// of memory traffic there, 4 TB/s, for 0.13 GB of fields).  The
 // launches per two iterations it replaces where a domain fits (k_sor_pair)
 // cost 8 us each on the smallest domains and recompute a four-cell ring and
 // six extra levels per block on large ones (0.37 of their lane-steps are
 // useful at 300x300x90).  Microseconds of a 50-iteration solve, before and
 // now: 24x20x16 455 and 163, 96x96x64 498 and 232, 150x150x90 675 and 319,
 // 203x117x61 878 and 318 (odd jm: one iteration per launch before), 256x256x64
-// 898 and 385, 300x300x90 1130 and 658.
+// 898 and 385, 300x300x90 1130 and 656.
 //
 // Waiting on other blocks is safe only while all of them run.  The blocks
 // first count themselves in (res_arrive, res_enter).  When all have arrived, none can be
 // left unscheduled and the waits always end.  When they have not within
-// kEnterTicks (another process's blocks hold the compute units), the launch
+// kEnterTicks (another process's blocks hold the compute units; the steps of
+// this one are in order, turns.h), the launch
 // falls back to sweeps over memory handed out by a ticket counter
 // (res_ticket): a sweep waits only for tickets taken earlier, which running
-// blocks hold, so that needs no co-residency at all.
+// blocks hold, so that needs no co-residency at all.  It takes 8 to 10 times
+// as long as the launch-per-iterations kernels, so the host, told by a counter,
+// goes over to those for some steps (res_review).
 #include <algorithm>
 #include <type_traits>
 

@@ -2216,9 +2216,9 @@ int les_domain_time_sor(les_domain* D, int iters, double* us_per_iter) {
 
 // ------------------------------------------------------------ batches
 // Several domains advanced together.  Domains whose whole step can be
-// batched run every stage as one launch for all of them and the SOR
-// iterations 2..nmaxp as one launch per iteration (k_sor_iter2_batch), on
-// the batch's stream; the others step whole on their own streams, joined by
+// batched run every stage as one launch for all of them, and the SOR as one
+// (k_sor_res, side by side) or its iterations 2..nmaxp as one launch per
+// iteration (k_sor_iter2_batch), on the batch's stream; the others step whole on their own streams, joined by
 // events.  Steps with every n > 1 replay one graph.
 
 int les_domain_set_graph(les_domain* D, int on) {
@@ -2575,10 +2575,12 @@ int batch_prepare(les_batch* B) {
 // domains batched by stage never enter the graph's streams: the graph runs
 // on the batch stream, and les_batch_step orders it against their streams.
 //  * Staged (every full domain at n > 1): the full domains' stages run as one
-//    launch per stage on the batch stream, their SOR iterations 2..nmaxp as
-//    one launch per iteration; the other domains step whole on their streams.
-//  * Otherwise (a first step): every full domain runs its stages and SOR
-//    iteration 1 on its own stream, the batched SOR iterations, then its own
+//    launch per stage on the batch stream, their SOR in one launch or, of those
+//    that do not solve so, iterations 2..nmaxp as one launch per iteration; the
+//    other domains step whole on their streams.
+//  * Otherwise (a first step): every full domain that solves in one launch
+//    steps whole on its own stream, one after the other; every other one runs its
+//    stages and SOR iteration 1 there, the batched SOR iterations, then its own
 //    press tail.
 int batch_enqueue(les_batch* B, const int* ns, const int* nmaxs, bool capturing) {
   const size_t nd = B->doms.size();

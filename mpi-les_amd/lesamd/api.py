@@ -386,8 +386,8 @@ class Domain:
 
 class Batch:
     """Domains advanced together (les_batch_*): one step of each per call,
-    every stage one launch for all of them and the SOR iterations one launch
-    per iteration."""
+    every stage one launch for all of them, and so the SOR of the domains that
+    solve in one launch, or each of its iterations."""
 
     def __init__(self, domains, graph: bool = True):
         self.domains = list(domains)

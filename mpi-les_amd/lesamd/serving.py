@@ -254,8 +254,8 @@ class Server:
     def run_batched(self, requests, max_batch_cells: int | None = None) -> list[Result]:
         """Continuous batching: the admitted domains of at most
         max_batch_cells cells (all of them when None) advance in lockstep, one
-        batched step (one launch per stage and per SOR iteration for all of
-        them) at a time, on the batch's stream; larger domains, which fill the
+        batched step (one launch per stage, and for the SOR or each of its
+        iterations, for all of them) at a time, on the batch's stream; larger domains, which fill the
         GPU by themselves, replay their own step graphs on their own streams
         alongside.  Requests join at step boundaries once their domain is
         ready, and leave when their last step has completed."""
