@@ -21,6 +21,7 @@
 
 #include "../../include/les_amd.h"
 #include "les_kernels.h"
+#include "solve_age.h"
 #include "turns.h"
 
 using namespace les;
@@ -498,6 +499,8 @@ struct les_domain {
   // seen so far, and where the domain stands after one (res_review).
   int res_want = 0, res_seen = 0;
   ResPause res_pause;
+  long long solves = 0;  // enqueued, of any kind
+  SolveAge res_age;      // of DevDomain::res_mem
 };
 
 namespace {
@@ -877,6 +880,17 @@ void res_review(les_domain* D) {
   } else if (P.length > 0 && ++P.good > P.length) {
     P.length = 0;
   }
+}
+
+// Before a press of D is enqueued: which form it takes, and its solves counted.
+// own: it may use the domain's own workspace.
+int press_begin(les_domain* D, bool own = true) {
+  res_review(D);
+  const int count = 1 + (D->d.press_mode == 1 ? D->d.dc_outer : 0);
+  D->solves += count;
+  if (own && press_resident(D->d) && D->res_age.use(D->solves, count))
+    HIP_TRY(hipMemsetAsync(D->d.res_mem, 0, (size_t)res_words(D->d.res) * 8, D->d.stream));
+  return 0;
 }
 
 void timer_free(les_domain* D) {
@@ -1739,7 +1753,7 @@ int les_press(int km, int jm, int im, float* rhs, const float* u, const float* d
   D->d.pjuge = pjuge_default;
   D->d.omega = omega_default;
   if (flush_metrics(D)) return 1;
-  res_review(D);
+  if (press_begin(D)) return 1;
   Turn turn(press_resident(D->d), D->d.stream);
   HIP_TRY(turn.err);
   return run_stage(D, 6, n, nmax);
@@ -2083,7 +2097,7 @@ int les_domain_destroy(les_domain* D) {
 int les_domain_stage(les_domain* D, int stage, int n, int nmax) {
   if (!live_has(D)) return fail("null, unknown or destroyed domain");
   if (flush_metrics(D)) return 1;
-  if (stage == 6) res_review(D);
+  if (stage == 6 && press_begin(D)) return 1;
   Turn turn(stage == 6 && press_resident(D->d), D->d.stream);
   HIP_TRY(turn.err);
   return run_stage(D, stage, n, nmax);
@@ -2131,7 +2145,7 @@ static int step_capture(les_domain* D, int n, int nmax) {
 int les_domain_step(les_domain* D, int n, int nmax) {
   if (!live_has(D)) return fail("null, unknown or destroyed domain");
   if (flush_metrics(D)) return 1;  // may allow or rule out the one-launch SOR
-  res_review(D);
+  if (press_begin(D)) return 1;
   const bool replay = D->use_graph && n != 1 && !D->d.timer;
   if (replay && step_capture(D, n, nmax)) return 1;
   Turn turn(press_resident(D->d), D->d.stream);
@@ -2340,6 +2354,9 @@ struct les_batch {
   std::vector<char> res;
   std::vector<ResBatch> res_launch;
   void* res_mem = nullptr;
+  char* res_work = nullptr;       // the workspaces in it, and their bytes
+  size_t res_work_bytes = 0;
+  std::vector<SolveAge> res_age;  // by domain, of its part
   void* stage_mem = nullptr;      // device: BatchDom[nfull], then StageSpan[BS_N][nfull]
   StageBatch stages{};            // stages.nd == 0: no batched stages
   std::vector<DevDomain> key;     // domain states the table and graph were made for
@@ -2451,9 +2468,29 @@ int batch_res_prepare(les_batch* B) {
     }
     B->res_launch.push_back(L);
   }
-  HIP_TRY(hipMemsetAsync(base + ntab + nb0, 0, 8 * words, B->stream));
+  B->res_work = base + ntab + nb0;
+  B->res_work_bytes = 8 * words;
+  B->res_age.assign(n, SolveAge());
+  for (size_t q = 0; q < n; q++) B->res_age[q].cleared(B->doms[q]->solves - 1);  // this step's is counted
+  HIP_TRY(hipMemsetAsync(B->res_work, 0, B->res_work_bytes, B->stream));
   HIP_TRY(copy_sync(base, tab.data(), tab.size() * sizeof(ResArgs), hipMemcpyHostToDevice, B->stream));
   HIP_TRY(copy_sync(base + ntab, b0s.data(), b0s.size() * sizeof(int), hipMemcpyHostToDevice, B->stream));
+  return 0;
+}
+
+// Clears the workspaces this step may use whose words may be too old.
+int batch_clear_aged(les_batch* B) {
+  bool clear = false;
+  for (size_t q = 0; q < B->doms.size(); q++) {
+    les_domain* D = B->doms[q];
+    if (B->res[q] && B->res_age[q].use(D->solves, 1)) clear = true;
+    const int count = 1 + (D->d.press_mode == 1 ? D->d.dc_outer : 0);  // a first step, or one on its own stream
+    if (press_resident(D->d) && D->res_age.use(D->solves, count))
+      HIP_TRY(hipMemsetAsync(D->d.res_mem, 0, (size_t)res_words(D->d.res) * 8, D->d.stream));
+  }
+  if (!clear) return 0;
+  for (size_t q = 0; q < B->doms.size(); q++) B->res_age[q].cleared(B->doms[q]->solves - 1);
+  HIP_TRY(hipMemsetAsync(B->res_work, 0, B->res_work_bytes, B->stream));
   return 0;
 }
 
@@ -2710,7 +2747,7 @@ int les_batch_step(les_batch* B, const int* ns, const int* nmaxs) {
   // a pause of one domain is one of the batch, the longest of theirs
   const les_domain* paused = nullptr;
   for (les_domain* D : B->doms) {
-    res_review(D);
+    if (press_begin(D, false)) return 1;
     if (D->res_pause.phase != 0 && (!paused || D->res_pause.rest > paused->res_pause.rest)) paused = D;
   }
   for (les_domain* D : B->doms)
@@ -2735,6 +2772,7 @@ int les_batch_step(les_batch* B, const int* ns, const int* nmaxs) {
     whole = whole || B->res[q] || (!B->full[q] && press_resident(B->doms[q]->d));
   bool replay = B->use_graph != 0;
   for (size_t q = 0; q < B->doms.size(); q++) replay = replay && ns[q] != 1;
+  if (batch_clear_aged(B)) return 1;
   if (replay && !B->gexec) {
     for (les_domain* D : B->doms)
       if (!D->d.fuse_velfg && ensure_cov(D)) return 1;  // allocations cannot be captured
